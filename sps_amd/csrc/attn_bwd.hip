@@ -9,10 +9,10 @@
 //       P = exp2(S*scale2 - LSE) (one fp32 FMA per score, as the reference scales its fp32 scores:
 //       triton_sps_flash_attention.py:471), dS = P (dP - Delta)   (lane-local LSE and Delta),
 //       dQ^T += K^T dS^T  (K^T fragments via ds_read_b64_tr_b16).
-//  2. dK/dV pass (key-stationary). A workgroup owns 128 keys of one stream (natural, persistent
-//     or temporary), each wave 32 of them held in registers; it walks the 32-query chunks of the
-//     union of its lanes' query intervals (persistent keys: diagonal to document end; temporary
-//     keys: the w-token window):
+//  2. dK/dV pass (key-stationary; head dims up to 64, attn_bwd_split.hip has the larger ones). A
+//     workgroup owns 128 keys of one stream (natural, persistent or temporary), each wave 32 of them
+//     held in registers; it walks the 32-query chunks of the union of its lanes' query intervals
+//     (persistent keys: diagonal to document end; temporary keys: the w-token window):
 //       S = Q K^T, dP = dO V^T (Q, dO rows from LDS; K, V in registers),
 //       P = exp2(S*scale2 - LSE) (fp32 FMA per score, triton_sps_flash_attention.py:361),
 //       dV^T += dO^T P, dK^T += Q^T dS (dO^T, Q^T fragments via ds_read_b64_tr_b16).
@@ -323,7 +323,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(bwd_waves<D
   // Head dims of 64 and more stage Q / dO chunks and their seeds by direct global -> LDS loads into
   // dense swizzled tiles; smaller ones through registers into padded tiles.
   constexpr bool kDma = D >= 64;
-  using DT = DmaTile<kDma ? D : 64, D != 256>;  // D = 256: the register-lean swizzle (fewer spills)
+  using DT = DmaTile<64>;
   constexpr bool kSkew = D == 64 && NG == 4;
   constexpr int kSkewMaxChunks = 16;
   constexpr int TE = kDma ? DT::ELEMS : G::ELEMS;
@@ -343,10 +343,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(bwd_waves<D
   const RowView row = row_view(a, b, tp.mono);
   KState st;
   int run_end;
-  // (The f16 dK/dV kernel at D = 256 keeps the span reductions: with the four-lane reads the
-  // compiler's AGPR-copy rewrite crashes on it.)
-  constexpr bool kMono = D != 256;
-  const bool planned = k_begin<kMono>(a, tp, row, s_span, st, run_end);
+  const bool planned = k_begin(a, tp, row, s_span, st, run_end, tid >> 6);
   const int kp = st.kp;
   const bool kvalid = st.kvalid;
   const int nc = st.nc;
@@ -466,7 +463,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(bwd_waves<D
       issue_regs(0, 0);
     if constexpr (kSkew)
       if (skew) issue_dma(1, 1);
-    if (planned) k_lanes<kMono>(m, run_end, st);
+    if (planned) k_lanes(m, run_end, st);
     // The dP tile starts from the -Delta seeds of its query rows, so it comes out of the MFMAs as
     // dP - Delta and dS = P * dP' is one VALU operation per element; the S tile is scaled in fp32 by
     // one FMA per score with the -LSE seeds (S * scale2 - LSE), never by rounding a scaled K.
@@ -657,7 +654,7 @@ __global__ __launch_bounds__(256) void mask_dump_kv_kernel(const AttnArgs a) {
   const RowView row = row_view(a, b, tp.mono);
   KState st;
   int run_end;
-  if (k_begin(a, tp, row, s_span, st, run_end)) k_lanes(m, run_end, st);
+  if (k_begin(a, tp, row, s_span, st, run_end, tid >> 6)) k_lanes(m, run_end, st);
   const bool exact = row.mono;
   const int64_t dk_doc = (!exact && st.kvalid) ? load_doc(a, b, st.kp) : 0;
   const BlockMask bm = k_block_mask(st, exact);
@@ -693,8 +690,13 @@ static hipError_t launch_bwd_t(const AttnArgs& a, int passes, hipStream_t stream
     if (e != hipSuccess) return e;
   }
   if ((passes & kBwdDkdv) && nk > 0) {
-    hipLaunchKernelGGL((attn_bwd_dkdv_kernel<D, E>), dim3((unsigned)nk), dim3(256), 0, stream, a);
-    return hipGetLastError();
+    // From D = 128 on a wave cannot hold K, V, dK and dV of 32 keys beside another wave: two share them.
+    if constexpr (D >= 128) {
+      return launch_attn_bwd_dkdv_split(a, D, std::is_same<E, ElemF16>::value, nk, stream);
+    } else {
+      hipLaunchKernelGGL((attn_bwd_dkdv_kernel<D, E>), dim3((unsigned)nk), dim3(256), 0, stream, a);
+      return hipGetLastError();
+    }
   }
   return hipSuccess;
 }

@@ -183,35 +183,10 @@ struct WaveSpan {
   int max_lo, min_hi;  // every lane's interval contains [max_lo, min_hi] (lanes with nothing break it)
 };
 
-// Reduction of x over the 64 lanes (all active) with an associative, commutative op; the result is
-// wave-uniform. Inside each row of 16 lanes by DPP moves (VALU, no LDS round trip): quad swaps, then
-// the half-row and row mirrors leave every lane of a row holding the row's result; the four rows
-// are then combined from one lane each.
-template <class Op>
-__device__ __forceinline__ int wave_reduce(int x, Op op) {
-  x = op(x, __builtin_amdgcn_mov_dpp(x, 0xB1, 0xF, 0xF, false));   // quad_perm [1, 0, 3, 2]
-  x = op(x, __builtin_amdgcn_mov_dpp(x, 0x4E, 0xF, 0xF, false));   // quad_perm [2, 3, 0, 1]
-  x = op(x, __builtin_amdgcn_mov_dpp(x, 0x141, 0xF, 0xF, false));  // row_half_mirror
-  x = op(x, __builtin_amdgcn_mov_dpp(x, 0x140, 0xF, 0xF, false));  // row_mirror
-  const int r0 = __builtin_amdgcn_readlane(x, 0), r1 = __builtin_amdgcn_readlane(x, 16);
-  const int r2 = __builtin_amdgcn_readlane(x, 32), r3 = __builtin_amdgcn_readlane(x, 48);
-  return op(op(r0, r1), op(r2, r3));
-}
-
-__device__ __forceinline__ WaveSpan wave_span(const Interval& r) {
-  const bool empty = r.lo > r.hi;
-  WaveSpan w;  // the reductions are wave-uniform: keep them in scalar registers
-  w.min_lo = __builtin_amdgcn_readfirstlane(wave_reduce(empty ? kEmptyLo : r.lo, [](int x, int y) { return imin(x, y); }));
-  w.max_hi = __builtin_amdgcn_readfirstlane(wave_reduce(empty ? kEmptyHi : r.hi, [](int x, int y) { return imax(x, y); }));
-  w.max_lo = __builtin_amdgcn_readfirstlane(wave_reduce(empty ? kEmptyLo : r.lo, [](int x, int y) { return imax(x, y); }));
-  w.min_hi = __builtin_amdgcn_readfirstlane(wave_reduce(empty ? kEmptyHi : r.hi, [](int x, int y) { return imin(x, y); }));
-  return w;
-}
-
-// The same spans for intervals that never decrease along the lanes 0-31 (lanes 32-63 repeat them):
+// A wave's spans from intervals that never decrease along the lanes 0-31 (lanes 32-63 repeat them):
 // the union runs from the first non-empty lane's lo to the last non-empty lane's hi, and the common
 // part, when no lane is empty, from lane 31's lo to lane 0's hi; four lane reads instead of four
-// reductions. The kernels' lanes hold consecutive queries (keys) of one stream, and both bounds of
+// reductions over the wave. The kernels' lanes hold consecutive queries (keys) of one stream, and both bounds of
 // their intervals are non-decreasing in the position (run starts and ends, the diagonal and the
 // window bounds all are).
 __device__ __forceinline__ WaveSpan wave_span_monotone(const Interval& r) {

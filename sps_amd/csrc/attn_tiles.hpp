@@ -87,12 +87,12 @@ struct TileRegs {
 // Dense LDS tile filled by direct global -> LDS loads (head dims of 64 and more): 32 rows of D
 // elements, no padding; the 16-byte chunks of each row are permuted by a row-dependent swizzle
 // instead (swz below).
-template <int D, bool kSpread = true>
+template <int D, bool kSpread = true, int THREADS = 256>
 struct DmaTile {
   static_assert(D == 64 || D % 128 == 0, "the swizzle permutes 8 chunks of a row at D = 64, 16 above");
   static constexpr int CPR = D / 8;                  // 16-byte chunks per row
   static constexpr int ELEMS = kBlock * D;           // one staged tile
-  static constexpr int PASSES = ELEMS / (256 * 8);   // 16-byte pieces per thread (1 for D = 64)
+  static constexpr int PASSES = ELEMS / (THREADS * 8);  // 16-byte pieces per thread (1 for D = 64 and 256 threads)
 
   // Logical chunk k of row r is stored at chunk k ^ swz(r), so that both fragment reads below hit
   // distinct LDS banks (64 banks of 4 bytes): a row-fragment b128 read gives 16 lanes 16 consecutive
@@ -114,7 +114,7 @@ struct DmaTile {
   }
 
   // Byte offsets, from the tile's first row, of the pieces thread tid loads: piece p fills slot
-  // p * 256 + tid of the tile (row slot / CPR, stored chunk slot % CPR).
+  // p * THREADS + tid of the tile (row slot / CPR, stored chunk slot % CPR).
   struct Src {
     uint32_t o[PASSES];
   };
@@ -122,7 +122,7 @@ struct DmaTile {
     Src s;
 #pragma unroll
     for (int p = 0; p < PASSES; ++p) {
-      const int slot = p * 256 + tid, r = slot / CPR, c = (slot % CPR) ^ swz(r);
+      const int slot = p * THREADS + tid, r = slot / CPR, c = (slot % CPR) ^ swz(r);
       s.o[p] = (uint32_t)r * row_step_bytes + (uint32_t)c * 16u;
     }
     return s;
@@ -132,7 +132,7 @@ struct DmaTile {
   // per piece and wave, each filling the wave's contiguous 1 KiB of the tile).
   static __device__ __forceinline__ void load(BufRsrc rs, uint32_t first, const Src& s, uint16_t* tile, int wave) {
 #pragma unroll
-    for (int p = 0; p < PASSES; ++p) lds_dma_b128(rs, tile + (p * 256 + wave * 64) * 8, first + s.o[p]);
+    for (int p = 0; p < PASSES; ++p) lds_dma_b128(rs, tile + (p * THREADS + wave * 64) * 8, first + s.o[p]);
   }
 
   // Element offset of row c32's chunk 2c + g (row-major fragment: 8 consecutive columns 16c + 8g).
@@ -217,11 +217,13 @@ __device__ __forceinline__ uint32_t qs_exact_bits(const AttnArgs& a, int b, cons
 }
 
 // Key-stationary exact visibility bits for a lane owning key kp (document id dk, last visible query
-// qhi) and the query chunk starting at position qc.
+// qhi) and the query chunk starting at position qc. UNROLL: id loads in flight at once (fewer
+// where a kernel is short of registers).
+template <int UNROLL = 16>
 __device__ __forceinline__ uint32_t ks_exact_bits(const AttnArgs& a, int b, int kp, int qhi, int qc, int g,
                                                   int64_t dk) {
   uint32_t bits = 0;
-#pragma unroll
+#pragma unroll UNROLL
   for (int i = 0; i < 16; ++i) {
     const int q = qc + acc_row(i, g);
     bool vis = q >= kp && q <= qhi;
@@ -351,9 +353,10 @@ struct KState {
   int c0, nc;
 };
 
-// The lane's key of key tile kt (lanes 32-63 repeat lanes 0-31).
-__device__ __forceinline__ void k_lane_key(const MaskSpec& m, int kt, KState& st) {
-  const int tid = threadIdx.x, wave = tid >> 6, c32 = tid & 31;
+// The lane's key of key tile kt (lanes 32-63 repeat lanes 0-31) in a wave that owns the tile's keys
+// 32 wave .. 32 wave + 31.
+__device__ __forceinline__ void k_lane_key(const MaskSpec& m, int kt, KState& st, int wave) {
+  const int c32 = threadIdx.x & 31;
   k_tile_run(m, kt, st.stream, st.first);
   const int t = st.first + wave * kBlock + c32;
   st.kvalid = t < stream_len(m.family, m.N, st.stream, m.P);
@@ -361,8 +364,6 @@ __device__ __forceinline__ void k_lane_key(const MaskSpec& m, int kt, KState& st
 }
 
 // The lane's query interval and the wave span, given the end e of the key's document run.
-// kMonotone: the span from four lane reads (wave_span_monotone), else from four reductions.
-template <bool kMonotone = true>
 __device__ __forceinline__ void k_lanes(const MaskSpec& m, int e, KState& st) {
   if (st.kvalid) {
     st.r.lo = st.kp;
@@ -371,13 +372,12 @@ __device__ __forceinline__ void k_lanes(const MaskSpec& m, int e, KState& st) {
   } else {
     st.r = Interval{kEmptyLo, kEmptyHi};
   }
-  st.w = kMonotone ? wave_span_monotone(st.r) : wave_span(st.r);
+  st.w = wave_span_monotone(st.r);
 }
 
 // Query chunks covering the union of the workgroup's lane intervals (one LDS exchange and barrier).
-__device__ __forceinline__ void k_plan_from_spans(int* s_span, KState& st) {
-  const int tid = threadIdx.x, wave = tid >> 6;
-  if ((tid & 63) == 0) {
+__device__ __forceinline__ void k_plan_from_spans(int* s_span, KState& st, int wave) {
+  if ((threadIdx.x & 63) == 0) {
     s_span[2 * wave + 0] = st.w.min_lo;
     s_span[2 * wave + 1] = st.w.max_hi;
   }
@@ -393,24 +393,22 @@ __device__ __forceinline__ void k_plan_from_spans(int* s_span, KState& st) {
   st.nc = wave_uniform(st.nc);
 }
 
-template <bool kMonotone = true>
-__device__ __forceinline__ void k_setup(const AttnArgs& a, const RowView& row, int kt, int* s_span, KState& st) {
-  k_lane_key(a.m, kt, st);
-  k_lanes<kMonotone>(a.m, st.kvalid ? row.run_end(st.kp, a.m.N) : 0, st);
-  k_plan_from_spans(s_span, st);
+__device__ __forceinline__ void k_setup(const AttnArgs& a, const RowView& row, int kt, int* s_span, KState& st, int wave) {
+  k_lane_key(a.m, kt, st, wave);
+  k_lanes(a.m, st.kvalid ? row.run_end(st.kp, a.m.N) : 0, st);
+  k_plan_from_spans(s_span, st, wave);
 }
 
 // Start of a key-stationary workgroup; as q_begin, with the lane's run end read here and consumed by
 // k_lanes(m, run_end, st) after the caller's first loads are issued.
-template <bool kMonotone = true>
 __device__ __forceinline__ bool k_begin(const AttnArgs& a, const TilePlan& tp, const RowView& row, int* s_span,
-                                        KState& st, int& run_end) {
+                                        KState& st, int& run_end, int wave) {
   run_end = 0;
   if (tp.n0 < 0) {
-    k_setup<kMonotone>(a, row, tp.tile, s_span, st);
+    k_setup(a, row, tp.tile, s_span, st, wave);
     return false;
   }
-  k_lane_key(a.m, tp.tile, st);
+  k_lane_key(a.m, tp.tile, st, wave);
   st.c0 = tp.b0;
   st.nc = tp.n0;
   if (st.kvalid) run_end = row.run_end(st.kp, a.m.N);

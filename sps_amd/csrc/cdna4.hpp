@@ -178,6 +178,12 @@ __device__ __forceinline__ void lds_dma_b32(BufRsrc r, float* lds, uint32_t voff
 // for registers loaded before the loop.
 __device__ __forceinline__ void vmem_wait_all() { __builtin_amdgcn_s_waitcnt(0x0F70); }
 
+// Workgroup barrier behind the wave's own LDS operations only: direct global -> LDS loads stay in
+// flight across it (a workgroup fence would wait for them).
+__device__ __forceinline__ void lds_only_barrier() {
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+}
+
 // Reads a value that is uniform across the wave into a scalar register.
 __device__ __forceinline__ int wave_uniform(int x) { return __builtin_amdgcn_readfirstlane(x); }
 
