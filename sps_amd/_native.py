@@ -183,6 +183,23 @@ def lib() -> C.CDLL:
     return _lib
 
 
+_binding = None
+
+
+def binding():
+    """The torch binding (csrc/torch_binding.cpp): the entry points' host path for ordinary eager calls.
+    Each of its functions returns None (kv_update: False) for a call it does not take."""
+    global _binding
+    if _binding is None:
+        lib()
+        try:
+            from . import _torch_binding
+        except ImportError as e:
+            raise ImportError("sps_amd: the torch binding is missing; build it with `python -m sps_amd.build`") from e
+        _binding = _torch_binding
+    return _binding
+
+
 def last_error() -> str:
     buf = C.create_string_buffer(1024)
     lib().sps_last_error(buf, len(buf))

@@ -238,6 +238,12 @@ _attention_fwd_op.register_autograd(_attention_backward, setup_context=_attentio
 
 
 def _attention(q, k, v, sm_scale, family, window, documents_idx_BxT, persistent_key_window):
+    # Ordinary eager calls run in native code from here on; what needs the registered ops (tracing,
+    # transforms, modes), a copy of an input or an error message comes back as None.
+    if not torch.compiler.is_compiling():
+        o = N.binding().attention(q, k, v, sm_scale, family, window, documents_idx_BxT, persistent_key_window)
+        if o is not None:
+            return o
     _validate(q, k, v, family, documents_idx_BxT)
     keep = torch.is_grad_enabled() and any(t.requires_grad for t in (q, k, v))
     o, _, _ = torch.ops.sps_amd.attention_fwd(

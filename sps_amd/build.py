@@ -1,4 +1,4 @@
-"""Builds libsps_attn.so (gfx950) in-tree with hipcc.
+"""Builds libsps_attn.so (gfx950) in-tree with hipcc, and the torch binding beside it with g++.
 
 Every HIP translation unit under ``sps_amd/csrc`` is compiled to an object in ``sps_amd/_build`` and
 linked into ``sps_amd/libsps_attn.so``. Run ``python -m sps_amd.build`` (or ``__graft_entry__.build()``).
@@ -11,12 +11,16 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 from pathlib import Path
+
+import torch
 
 PKG_DIR = Path(__file__).resolve().parent
 CSRC = PKG_DIR / "csrc"
 BUILD_DIR = PKG_DIR / "_build"
 LIB_PATH = PKG_DIR / "libsps_attn.so"
+BINDING_PATH = PKG_DIR / "_torch_binding.so"
 ARCH = "gfx950"
 
 HIP_FLAGS = [
@@ -66,18 +70,46 @@ def _compile(hipcc: str, src: Path, obj: Path) -> None:
         raise RuntimeError(f"hipcc failed for {src.name}:\n{proc.stderr}")
 
 
+def _compile_binding(obj: Path) -> None:
+    """The torch binding's object: host code only (g++, torch and HIP headers)."""
+    from torch.utils import cpp_extension
+
+    includes = [*cpp_extension.include_paths(), "/opt/rocm/include", sysconfig.get_paths()["include"]]
+    cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-DUSE_ROCM", "-D__HIP_PLATFORM_AMD__=1",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch.compiled_with_cxx11_abi())}",
+           *(f"-isystem{p}" for p in includes), "-c", str(CSRC / "torch_binding.cpp"), "-o", str(obj)]
+    proc = subprocess.run(cmd, capture_output=True, text=True)
+    if proc.returncode != 0:
+        raise RuntimeError(f"g++ failed for torch_binding.cpp:\n{proc.stderr}")
+
+
+def _link_binding(obj: Path) -> None:
+    from torch.utils import cpp_extension
+
+    tmp = BINDING_PATH.with_suffix(".so.tmp")
+    cmd = [os.environ.get("CXX", "g++"), "-shared", str(obj), "-o", str(tmp), f"-L{PKG_DIR}", "-l:libsps_attn.so",
+           *(f"-L{p}" for p in cpp_extension.library_paths()), "-ltorch", "-ltorch_cpu", "-ltorch_hip", "-lc10",
+           "-lc10_hip", "-ltorch_python", "-Wl,-rpath,$ORIGIN"]
+    proc = subprocess.run(cmd, capture_output=True, text=True)
+    if proc.returncode != 0:
+        raise RuntimeError(f"linking the torch binding failed:\n{proc.stderr}")
+    os.replace(tmp, BINDING_PATH)
+
+
 def build(verbose: bool = False) -> Path:
     """Compiles every source and links the shared library; returns its path."""
     hipcc = _hipcc()
     BUILD_DIR.mkdir(exist_ok=True)
     objs = []
-    with cf.ThreadPoolExecutor(max_workers=min(len(SOURCES), os.cpu_count() or 4)) as ex:
+    with cf.ThreadPoolExecutor(max_workers=min(len(SOURCES) + 1, os.cpu_count() or 4)) as ex:
         futs = {}
         for name in SOURCES:
             src = CSRC / name
             obj = BUILD_DIR / (src.stem + ".o")
             objs.append(obj)
             futs[ex.submit(_compile, hipcc, src, obj)] = name
+        binding_obj = BUILD_DIR / "torch_binding.o"
+        futs[ex.submit(_compile_binding, binding_obj)] = "torch_binding.cpp"
         for fut in cf.as_completed(futs):
             fut.result()
             if verbose:
@@ -88,8 +120,9 @@ def build(verbose: bool = False) -> Path:
     if proc.returncode != 0:
         raise RuntimeError(f"link failed:\n{proc.stderr}")
     os.replace(tmp, LIB_PATH)
+    _link_binding(binding_obj)
     if verbose:
-        print(f"[sps_amd.build] wrote {LIB_PATH}", flush=True)
+        print(f"[sps_amd.build] wrote {LIB_PATH} and {BINDING_PATH}", flush=True)
     return LIB_PATH
 
 

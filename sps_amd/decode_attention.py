@@ -196,6 +196,11 @@ def triton_segmented_q1_attention(
     reference's contract: the caller then falls back). ``_kv_update`` is internal
     (decode_attention_fast.segmented_q1_attention_with_kv_update).
     """
+    if _kv_update is None and not torch.compiler.is_compiling():
+        # Ordinary eager calls run in native code; None: the general path below.
+        out = N.binding().decode(q_BxHxD, 1, segments, extra_kv, attn_dtype, None)
+        if out is not None:
+            return out
     if not q_BxHxD.is_cuda:
         return None
     if len(segments) > 3:
@@ -235,6 +240,12 @@ def triton_segmented_q2_attention(
     (<predict>) additionally sees the current <predict> key. Fail-fast: raises RuntimeError on any
     unsupported input, as the reference does. Returns fp32 [B, 2, H, D]. ``_kv_update`` is internal
     (decode_attention_fast.segmented_q2_attention_with_kv_update)."""
+    if _kv_update is None and not torch.compiler.is_compiling():
+        out = N.binding().decode(q_Bx2xHxD, 2, segments, [(current_normal_k_BxHxD, current_normal_v_BxHxD),
+                                                          (current_predict_k_BxHxD, current_predict_v_BxHxD)],
+                                 attn_dtype, None)
+        if out is not None:
+            return out
     if not q_Bx2xHxD.is_cuda:
         raise RuntimeError("CUDA tensors are required for SPS-family cached generation attention")
     if len(segments) > 2:

@@ -136,6 +136,10 @@ def fused_sps_kv_update(
     window_tokens: int,
 ) -> None:
     """One-launch KV update of one decode layer (see the module docstring)."""
+    if not torch.compiler.is_compiling() and N.binding().kv_update((
+            nw_k, nw_v, nw_len, nw_pos, br_k, br_v, br_len, k_window_BxHxD, v_window_BxHxD, k_retained_BxHxD,
+            v_retained_BxHxD, active_mask_B, window_tokens)):
+        return
     run_kv_update(kv_update_args(
         nw_k=nw_k, nw_v=nw_v, nw_len=nw_len, nw_pos=nw_pos, br_k=br_k, br_v=br_v, br_len=br_len,
         k_window_BxHxD=k_window_BxHxD, v_window_BxHxD=v_window_BxHxD, k_retained_BxHxD=k_retained_BxHxD,
@@ -173,6 +177,14 @@ def segmented_q2_attention_with_kv_update(
     and lengths are updated in place. The caches must have the segments' dtype."""
     from .decode_attention import triton_segmented_q2_attention
 
+    if not torch.compiler.is_compiling():
+        out = N.binding().decode(
+            q_Bx2xHxD, 2, segments, [(current_normal_k_BxHxD, current_normal_v_BxHxD),
+                                     (current_predict_k_BxHxD, current_predict_v_BxHxD)], attn_dtype,
+            (nw_k, nw_v, nw_len, nw_pos, br_k, br_v, br_len, k_window_BxHxD, v_window_BxHxD, k_retained_BxHxD,
+             v_retained_BxHxD, active_mask_B, window_tokens))
+        if out is not None:
+            return out
     upd = kv_update_args(
         nw_k=nw_k, nw_v=nw_v, nw_len=nw_len, nw_pos=nw_pos, br_k=br_k, br_v=br_v, br_len=br_len,
         k_window_BxHxD=k_window_BxHxD, v_window_BxHxD=v_window_BxHxD, k_retained_BxHxD=k_retained_BxHxD,
@@ -209,6 +221,13 @@ def segmented_q1_attention_with_kv_update(
     fp32 [B, H, D]; raises RuntimeError where the q1 kernel does not apply (there is no other path)."""
     from .decode_attention import triton_segmented_q1_attention
 
+    if not torch.compiler.is_compiling():
+        out = N.binding().decode(
+            q_BxHxD, 1, segments, extra_kv, attn_dtype,
+            (nw_k, nw_v, nw_len, nw_pos, br_k, br_v, br_len, k_window_BxHxD, v_window_BxHxD, k_retained_BxHxD,
+             v_retained_BxHxD, active_mask_B, window_tokens))
+        if out is not None:
+            return out
     upd = kv_update_args(
         nw_k=nw_k, nw_v=nw_v, nw_len=nw_len, nw_pos=nw_pos, br_k=br_k, br_v=br_v, br_len=br_len,
         k_window_BxHxD=k_window_BxHxD, v_window_BxHxD=v_window_BxHxD, k_retained_BxHxD=k_retained_BxHxD,

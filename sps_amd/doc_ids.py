@@ -38,14 +38,14 @@ def document_ids(idx_BxT: Tensor, *, eos_token_id: int, pad_token_id: int, repea
     if out_dtype not in _INT_CODES:
         raise TypeError(f"document ids must be int32 or int64, got {out_dtype}")
     out = torch.empty((b, t * repeat), dtype=out_dtype, device=tok.device)
-    bad = torch.zeros((b,), dtype=torch.int32, device=tok.device) if validate else None
+    bad = torch.empty((b,), dtype=torch.int32, device=tok.device) if validate else None  # the kernel writes every flag
     status = N.lib().sps_document_ids(
         b, t, tok.data_ptr(), _INT_CODES[tok.dtype], tok.stride(0) if b > 1 else t, int(eos_token_id),
         int(pad_token_id), int(repeat), out.data_ptr(), _INT_CODES[out_dtype], out.stride(0) if b > 1 else t * repeat,
         bad.data_ptr() if bad is not None else None, torch.cuda.current_stream(tok.device).cuda_stream)
     N.check("sps_document_ids", status)
     if bad is not None:
-        rows = bad.nonzero().flatten().tolist()
+        rows = [i for i, flag in enumerate(bad.tolist()) if flag]
         if rows:
             raise ValueError(f"token rows {rows} are not left padded: a pad token follows a real token")
     return out

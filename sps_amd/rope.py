@@ -139,6 +139,10 @@ def _conj(freqs_cis: Tensor) -> Tensor:
 
 def apply_rotary_emb(xq: Tensor, xk: Tensor, freqs_cis: Tensor) -> Tuple[Tensor, Tensor]:
     """RoPE on [B, T, H, D] queries and keys; returns new tensors of the inputs' dtype and shape."""
+    if not torch.compiler.is_compiling():
+        outs = N.binding().rope(xq, xk, None, freqs_cis, None)
+        if outs is not None:
+            return outs
     assert xq.ndim == 4 and xk.shape == xq.shape
     return torch.ops.sps_amd.rope_pair(xq, xk, freqs_cis)
 
@@ -149,6 +153,10 @@ def rope_qkv_for_attention(q: Tensor, k: Tensor, v: Tensor, freqs_cis: Tensor,
     QKV projection are fine) -> RoPE(q), RoPE(k), v in ``out_dtype`` as [B, H, T, D] views of
     [B, T, H, D] buffers, ready for sps_sliding_attention / reverse_sps_sliding_attention /
     full_attention."""
+    if not torch.compiler.is_compiling():
+        outs = N.binding().rope(q, k, v, freqs_cis, out_dtype)
+        if outs is not None:
+            return outs
     assert q.ndim == 4 and k.shape == q.shape and v.shape == q.shape
     assert out_dtype in _FLOAT_DTYPES
     outs = torch.ops.sps_amd.rope_qkv(q, k, v, freqs_cis, out_dtype)
