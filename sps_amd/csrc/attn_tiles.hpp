@@ -202,11 +202,12 @@ __device__ __forceinline__ void mask_partial(f32x16_t& s, const Interval& r, con
 
 // Query-stationary exact visibility bits for a lane owning query qp (document id dq) and a block
 // of 32 indices of `stream` starting at t0, when the row's ids are arbitrary: interval test and
-// per-pair id equality.
+// per-pair id equality. UNROLL: id loads in flight at once (fewer where a kernel is short of registers).
+template <int UNROLL = 16>
 __device__ __forceinline__ uint32_t qs_exact_bits(const AttnArgs& a, int b, const Interval& r, int stream, int t0,
                                                   int g, int64_t dq) {
   uint32_t bits = 0;
-#pragma unroll
+#pragma unroll UNROLL
   for (int i = 0; i < 16; ++i) {
     const int t = t0 + acc_row(i, g);
     bool vis = t >= r.lo && t <= r.hi;
