@@ -308,7 +308,8 @@ static bool decode_head_dim(int D) { return D == 16 || D == 32 || D == 64 || D =
 
 size_t sps_decode_workspace_bytes(int B, int H, int D, int nq, int kv_dtype, int n_seg, const int64_t* seg_scan) {
   if (!decode_head_dim(D) || B < 0 || H < 0 || n_seg < 0 || n_seg > sps::kMaxDecodeSegs) return 0;
-  const int ck = sps::decode_chunk_keys(D, kv_bytes(kv_dtype));
+  const int kb = kv_bytes(kv_dtype);
+  const int ck = sps::decode_chunk_keys(D, kb, sps::decode_pass(B, H, D, kb, n_seg, seg_scan));
   int64_t chunks = 0;
   for (int s = 0; s < n_seg; ++s) chunks += (seg_scan[s] + ck - 1) / ck;
   const size_t bytes = (size_t)B * H * chunks * nq * sps::decode_record_floats(D) * sizeof(float);
@@ -360,7 +361,8 @@ static int decode_impl(int B, int H, int D, int nq, const void* q, int q_dtype, 
   a.n_extra = n_extra;
   const int kb = kv_bytes(kv_dtype);
   const int epl = 16 / kb;
-  const int ck = sps::decode_chunk_keys(D, kb);
+  const int pass = sps::decode_pass(B, H, D, kb, n_seg, seg_scan);
+  const int ck = sps::decode_chunk_keys(D, kb, pass);
   int chunk = 0;
   for (int s = 0; s < n_seg; ++s) {
     sps::DecodeSeg& sg = a.seg[s];
@@ -400,6 +402,8 @@ static int decode_impl(int B, int H, int D, int nq, const void* q, int q_dtype, 
   }
   a.n_chunks = chunk;
   a.chunk_keys = ck;
+  a.chunk_shift = __builtin_ctz((unsigned)ck);
+  a.pass = pass;
   for (int e = 0; e < n_extra; ++e) {
     if (!extra_k[e] || !extra_v[e]) return fail(SPS_E_INVALID, "extra %d: null pointer", e);
     a.ek[e] = extra_k[e];

@@ -70,6 +70,7 @@ __device__ __forceinline__ void unpack16(const u32x4_t w, float* out) {
 }
 
 __device__ __forceinline__ int imin_d(int x, int y) { return x < y ? x : y; }
+__device__ __forceinline__ int imax_d(int x, int y) { return x > y ? x : y; }
 
 __device__ __forceinline__ int seg_live_len(const DecodeSeg& sg, int b, int h, int H) {
   if (sg.scan == 0) return 0;
@@ -156,16 +157,15 @@ __device__ __forceinline__ void snapshot_lengths(const DecodeArgs& a, int b, int
 // Three waves per SIMD: the two-query form otherwise compiles to 170 VGPRs, one wave per SIMD fewer
 // than at 168, which measured 6 % slower at C5 (q = 2: 117.3 against 110.5 us); at D = 16 the
 // 168-register budget would spill 18 VGPRs, so that head dim keeps the compiler's choice.
-template <int D, int NQ, class KV, bool PQ>
+template <int D, int NQ, class KV, bool PQ, int PASS>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 16 ? 1 : 3, 8))) void decode_partial_kernel(
     const DecodeArgs a) {
   constexpr int EPL = 16 / (int)sizeof(typename KV::raw);  // elements per 16-byte load
   constexpr int LPR = D / EPL;                              // lanes per key row
   constexpr int RPP = 64 / LPR;                             // rows per wave pass
-  constexpr int PASS = DecodeGeom<D, sizeof(typename KV::raw)>::PASS;
   constexpr int KW = RPP * PASS;                            // keys per wave
   constexpr int CK = 4 * KW;                                // keys per workgroup chunk
-  static_assert(CK == DecodeGeom<D, sizeof(typename KV::raw)>::CHUNK, "chunk geometry");
+  static_assert(CK == DecodeGeom<D, sizeof(typename KV::raw), PASS>::CHUNK, "chunk geometry");
   __shared__ float s_m[4][NQ], s_l[4][NQ];
   __shared__ __attribute__((aligned(16))) float s_acc[4][NQ][D];
 
@@ -271,7 +271,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 16 ? 1
     }
   }
   __syncthreads();
-  constexpr int REC = DecodeGeom<D, 2>::REC;
+  constexpr int REC = decode_record_floats(D);
   float* out = a.part + (((int64_t)(b * a.H + h) * a.n_chunks + c) * NQ) * REC;
   for (int i = tid; i < NQ * D; i += 256) {
     const int qi = i / D, d = i - qi * D;
@@ -304,6 +304,14 @@ __device__ __forceinline__ int live_chunk(const DecodeArgs& a, const int* nc, in
   return -1;
 }
 
+// The value in scalar registers. Selects per lane among launch arguments go through this: otherwise the
+// compiler selects the argument's address and loads it per lane, one more memory round trip.
+template <class T>
+__device__ __forceinline__ T scalar(T x) {
+  asm volatile("" : "+s"(x));
+  return x;
+}
+
 template <int N>
 __device__ __forceinline__ float wave_max_f(float x) {
 #pragma unroll
@@ -312,16 +320,24 @@ __device__ __forceinline__ float wave_max_f(float x) {
 }
 
 // One wave per (query slot, head, batch): merges the chunk partials and the extra keys, normalises
-// and writes fp32. Everything that depends only on the chunk list is loaded in one round trip
-// before the max reduction: the extra keys' rows, each lane's chunk maximum and weight sum (lanes own
-// chunks, in rounds of 64), and the accumulator rows of the first kMergeAhead chunks (lanes over d).
-// Chunks beyond those are read 8 records per batch after the max is known.
-constexpr int kMergeAhead = 16;
+// and writes fp32. The launch is a chain of latencies (7.3 us for 16 x 12 or 64 x 16 (sequence, head)s
+// with the loads in dependent rounds, 6.2-6.9 us as here, MI355X), so everything is loaded in one round
+// trip before the max reduction: the extra keys' rows, each lane's chunk maximum and weight sum, and the accumulator
+// rows of the first chunks (lanes over d). DIRECT (at most 64 chunks, live or not): lane c owns chunk c,
+// so not even the lengths are needed to start the loads, and the records of chunks that turn out not
+// to be live are read and dropped; otherwise lanes own the live chunks in rounds of 64, after the
+// lengths. Chunks past those loaded ahead are read 8 records per batch once the max is known. WIDTH:
+// bytes per element of the query and the extras (0: they differ; the branch on the type then waits
+// for the loads before it).
+template <int D>
+constexpr int merge_ahead() { return D <= 128 ? 24 : 16; }
 
-template <int D, int NQ>
+template <int D, int NQ, bool DIRECT, int WIDTH>
 __global__ __launch_bounds__(64) void decode_merge_kernel(const DecodeArgs a) {
+  constexpr int kMergeAhead = merge_ahead<D>();
   constexpr int DPL = (D + 63) / 64;  // output elements per lane
-  constexpr int REC = DecodeGeom<D, 2>::REC;
+  constexpr int REC = decode_record_floats(D);
+  auto inside = [](int dd) { return D % 64 == 0 || dd < D; };  // lanes past D have no element
   const int qi = blockIdx.x, h = blockIdx.y, b = blockIdx.z, lane = threadIdx.x;
   // With the KV update folded in, lengths come from the snapshot only (this launch writes them).
   const int64_t* snap = a.snap ? a.snap + ((int64_t)b * a.H + h) * kSnapWords : nullptr;
@@ -330,66 +346,131 @@ __global__ __launch_bounds__(64) void decode_merge_kernel(const DecodeArgs a) {
   // V}, piece j), loaded first: nothing else depends on them, and they are stored at the end.
   constexpr int kUpdPieces = 4;  // per lane: 4 rows of at most 1 KiB (D = 256 in fp32)
   u32x4_t uval[kUpdPieces];
-  int upr = 0;
+  // Pieces per row: D / 8 (16-bit caches) or D / 4, a power of two.
+  const int upr_shift = __builtin_ctz(D / 8) + (a.upd.kv_dtype == 2 ? 1 : 0);
   if (upd) {
     const KvUpdateArgs& u = a.upd;
-    upr = u.D * (u.kv_dtype == 2 ? 4 : 2) / 16;
+    const int esz = u.kv_dtype == 2 ? 4 : 2;
+    auto row = [&](const void* p, int64_t sb, int64_t sh) {
+      return scalar(static_cast<const char*>(p) + (b * sb + h * sh) * esz);
+    };
+    const char* const kw = row(u.kw, u.kw_sb, u.kw_sh);
+    const char* const vw = row(u.vw, u.vw_sb, u.vw_sh);
+    const char* const kr = row(u.kr, u.kr_sb, u.kr_sh);
+    const char* const vr = row(u.vr, u.vr_sb, u.vr_sh);
 #pragma unroll
     for (int i = 0; i < kUpdPieces; ++i) {
-      const int pc = lane + 64 * i, r = pc / upr, j = pc - r * upr;
-      if (r < 4 && (r >= 2 || u.window > 0)) {
-        const void* src = r == 0 ? u.kw : r == 1 ? u.vw : r == 2 ? u.kr : u.vr;
-        const int64_t sb = r == 0 ? u.kw_sb : r == 1 ? u.vw_sb : r == 2 ? u.kr_sb : u.vr_sb;
-        const int64_t sh = r == 0 ? u.kw_sh : r == 1 ? u.vw_sh : r == 2 ? u.kr_sh : u.vr_sh;
-        const int esz = u.kv_dtype == 2 ? 4 : 2;
-        uval[i] = *reinterpret_cast<const u32x4_t*>(static_cast<const char*>(src) + (b * sb + h * sh) * esz + j * 16);
-      }
+      const int pc = lane + 64 * i, r = pc >> upr_shift, j = pc - (r << upr_shift);
+      if (r < 4 && (r >= 2 || u.window > 0))
+        uval[i] = *reinterpret_cast<const u32x4_t*>((r == 0 ? kw : r == 1 ? vw : r == 2 ? kr : vr) + j * 16);
     }
   }
+  const float* part = a.part + ((int64_t)(b * a.H + h) * a.n_chunks) * NQ * REC + qi * REC;
+  float m0 = 0.f, l0 = 0.f, x[kMergeAhead][DPL];
+  // The records of the lane's chunk c and of the first chunks (chunk(u): the u-th, in bounds for every u;
+  // unconditional loads, dropped where u is past the end).
+  auto load_records = [&](int c, auto chunk) {
+    const float* r0 = part + (int64_t)c * NQ * REC;
+    m0 = r0[D];
+    l0 = r0[D + 1];
+#pragma unroll
+    for (int u = 0; u < kMergeAhead; ++u) {
+      const int cu = chunk(u);
+      const float* ru = part + (int64_t)cu * NQ * REC;
+#pragma unroll
+      for (int i = 0; i < DPL; ++i) {
+        const int dd = lane + 64 * i;
+        x[u][i] = inside(dd) ? ru[dd] : 0.f;
+      }
+    }
+  };
+  if constexpr (DIRECT) {
+    const int last = a.n_chunks - 1;
+    if (last >= 0) load_records(imin_d(lane, last), [&](int u) { return imin_d(u, last); });
+  }
+  // The query slice and the extra keys' rows, as raw bits: converting a value where it is loaded would
+  // wait for each load in turn.
+  const int64_t q0 = b * a.q_sb + qi * a.q_ss + h * a.q_sh;
+  const int64_t e0 = b * a.e_sb + h * a.e_sh;
+  uint32_t qd[DPL], ekd[kMaxDecodeExtras][DPL], evd[kMaxDecodeExtras][DPL];
+  auto load_raw = [&](auto* q) {
+#pragma unroll
+    for (int i = 0; i < DPL; ++i) {
+      const int dd = lane + 64 * i;
+      qd[i] = inside(dd) ? (uint32_t)q[q0 + dd] : 0u;
+    }
+  };
+  auto load_raw_extras = [&](auto* type) {
+    using T = std::remove_pointer_t<decltype(type)>;
+#pragma unroll
+    for (int e = 0; e < kMaxDecodeExtras; ++e) {
+#pragma unroll
+      for (int i = 0; i < DPL; ++i) {
+        const int dd = lane + 64 * i;
+        const bool ld = e < a.n_extra && inside(dd);
+        ekd[e][i] = ld ? (uint32_t) reinterpret_cast<const T*>(a.ek[e])[e0 + dd] : 0u;
+        evd[e][i] = ld ? (uint32_t) reinterpret_cast<const T*>(a.ev[e])[e0 + dd] : 0u;
+      }
+    }
+  };
+  if (WIDTH == 4 || (WIDTH == 0 && a.q_dtype == 2))
+    load_raw(reinterpret_cast<const uint32_t*>(a.q));
+  else
+    load_raw(reinterpret_cast<const uint16_t*>(a.q));
+  if (WIDTH == 4 || (WIDTH == 0 && a.e_dtype == 2))
+    load_raw_extras(static_cast<uint32_t*>(nullptr));
+  else
+    load_raw_extras(static_cast<uint16_t*>(nullptr));
+  // The lengths, one per lane in one load: the snapshot's words, or each segment's length.
+  int64_t word = 0;
+  if (snap) {
+    if (lane < kSnapWords) word = snap[lane];
+  } else {
+    // Element idx of the lane's segment (segments without chunks have no length array).
+    auto element = [&](const DecodeSeg& sg) {
+      const int64_t idx = sg.len_per_head ? (int64_t)b * a.H + h : b;
+      return scalar(static_cast<const char*>(sg.len) + (sg.len ? idx * (sg.len_i64 ? 8 : 4) : 0));
+    };
+    const char* const l0 = element(a.seg[0]);
+    const char* const l1 = element(a.seg[1]);
+    const char* const l2 = element(a.seg[2]);
+    const int wide = scalar(a.seg[0].len_i64 | a.seg[1].len_i64 << 1 | a.seg[2].len_i64 << 2);
+    const char* const len = lane == 0 ? l0 : lane == 1 ? l1 : l2;
+    if (lane < a.n_seg && len) {
+      if ((wide >> lane) & 1)
+        word = *reinterpret_cast<const int64_t*>(len);
+      else
+        word = *reinterpret_cast<const int32_t*>(len);
+    }
+  }
+  auto snap_word = [&](int i) {
+    const uint32_t lo = __builtin_amdgcn_readlane((uint32_t)word, i);
+    const uint32_t hi = __builtin_amdgcn_readlane((uint32_t)((uint64_t)word >> 32), i);
+    return (int64_t)(((uint64_t)hi << 32) | lo);
+  };
   int nc[kMaxDecodeSegs] = {0, 0, 0};
   int total = 0;
   for (int s = 0; s < a.n_seg; ++s) {
-    const int live = snap ? (int)snap[s] : seg_live_len(a.seg[s], b, h, a.H);
-    nc[s] = (live + a.chunk_keys - 1) / a.chunk_keys;
+    const int64_t len = snap_word(s);
+    const int live = (int)(len < 0 ? 0 : len > a.seg[s].scan ? a.seg[s].scan : len);
+    nc[s] = (live + a.chunk_keys - 1) >> a.chunk_shift;
     total += nc[s];
   }
-  const float* part = a.part + ((int64_t)(b * a.H + h) * a.n_chunks) * NQ * REC + qi * REC;
-
-  // The query slice and the extra keys' rows.
-  const int64_t q0 = b * a.q_sb + qi * a.q_ss + h * a.q_sh;
-  const int64_t e0 = b * a.e_sb + h * a.e_sh;
-  float qd[DPL], ekd[kMaxDecodeExtras][DPL], evd[kMaxDecodeExtras][DPL];
+  // This lane's chunk of the first round (-1: none), the number of chunks of that round, and the lanes
+  // whose chunk is live.
+  int c0 = -1, nk;
+  if constexpr (DIRECT) {
 #pragma unroll
-  for (int i = 0; i < DPL; ++i) {
-    const int dd = lane + 64 * i;
-    qd[i] = dd < D ? load_as_f32(a.q, q0 + dd, a.q_dtype) : 0.f;
+    for (int s = 0; s < kMaxDecodeSegs; ++s)
+      if (s < a.n_seg && lane >= a.seg[s].chunk_base && lane < a.seg[s].chunk_base + nc[s]) c0 = lane;
+    nk = a.n_chunks;
+  } else {
+    nk = imin_d(64, total);
+    c0 = lane < total ? live_chunk(a, nc, lane) : -1;
+    // Idle lanes read chunk 0's record: in bounds.
+    load_records(c0 < 0 ? 0 : c0, [&](int u) { return imax_d(__shfl(c0, u), 0); });
   }
-#pragma unroll
-  for (int e = 0; e < kMaxDecodeExtras; ++e) {
-#pragma unroll
-    for (int i = 0; i < DPL; ++i) {
-      const int dd = lane + 64 * i;
-      const bool ld = e < a.n_extra && dd < D;
-      ekd[e][i] = ld ? load_as_f32(a.ek[e], e0 + dd, a.e_dtype) : 0.f;
-      evd[e][i] = ld ? load_as_f32(a.ev[e], e0 + dd, a.e_dtype) : 0.f;
-    }
-  }
-  // This lane's chunk of the first round (chunk 0's record for idle lanes: in bounds).
-  const int c0 = lane < total ? live_chunk(a, nc, lane) : -1;
-  const float* r0 = part + (int64_t)(c0 < 0 ? 0 : c0) * NQ * REC;
-  const float m0 = r0[D], l0 = r0[D + 1];
-  // Accumulator rows of the first kMergeAhead chunks.
-  float x[kMergeAhead][DPL];
-#pragma unroll
-  for (int u = 0; u < kMergeAhead; ++u) {
-    const int cu = __shfl(c0, u);
-    const float* ru = part + (int64_t)(cu < 0 ? 0 : cu) * NQ * REC;
-#pragma unroll
-    for (int i = 0; i < DPL; ++i) {
-      const int dd = lane + 64 * i;
-      x[u][i] = (u < total && dd < D) ? ru[dd] : 0.f;
-    }
-  }
+  const uint64_t live_lanes = __builtin_amdgcn_ballot_w64(c0 >= 0);
 
   // Extra-key scores (all lanes hold them after the reduction).
   float es[kMaxDecodeExtras] = {-INFINITY, -INFINITY};
@@ -398,14 +479,14 @@ __global__ __launch_bounds__(64) void decode_merge_kernel(const DecodeArgs a) {
     if (e >= a.n_extra) continue;
     float d = 0.f;
 #pragma unroll
-    for (int i = 0; i < DPL; ++i) d = fmaf(qd[i], ekd[e][i], d);
+    for (int i = 0; i < DPL; ++i) d = fmaf(raw_as_f32(qd[i], a.q_dtype), raw_as_f32(ekd[e][i], a.e_dtype), d);
     d = xor_sum<64>(d);
     if ((a.emask[e] >> qi) & 1) es[e] = d * a.scale2;
   }
 
   // Max over chunk maxima and extra scores.
   float M = fmaxf(fmaxf(es[0], es[1]), c0 >= 0 ? m0 : -INFINITY);
-  for (int k0 = 64; k0 < total; k0 += 64) {
+  for (int k0 = 64; !DIRECT && k0 < total; k0 += 64) {
     const int c = k0 + lane < total ? live_chunk(a, nc, k0 + lane) : -1;
     const float mc = part[(int64_t)(c < 0 ? 0 : c) * NQ * REC + D];  // in-bounds even for idle lanes
     M = fmaxf(M, c >= 0 ? mc : -INFINITY);
@@ -417,16 +498,20 @@ __global__ __launch_bounds__(64) void decode_merge_kernel(const DecodeArgs a) {
   float L = 0.f, A[DPL];
 #pragma unroll
   for (int i = 0; i < DPL; ++i) A[i] = 0.f;
-  // Accumulates the chunks [from, nk) of the round whose lane chunk / weight are (c, f).
-  auto accumulate = [&](int c, float f, int from, int nk) {
+  // Accumulates the chunks [from, nk) of the round whose lane chunk / weight are (c, f); live: bit j set
+  // where lane j's chunk is live (the others' records hold anything).
+  auto accumulate = [&](int c, float f, int from, int nk, uint64_t live) {
     for (int j0 = from; j0 < nk; j0 += 8) {
+      if (((live >> j0) & 0xff) == 0) continue;
       float fj[8];
       const float* rj[8];
+      bool on[8];
 #pragma unroll
       for (int u = 0; u < 8; ++u) {
         const int j = imin_d(j0 + u, nk - 1);
-        fj[u] = j0 + u < nk ? __shfl(f, j) : 0.f;
-        const int cj = __shfl(c, j);
+        on[u] = j0 + u < nk && ((live >> j) & 1);
+        fj[u] = on[u] ? __shfl(f, j) : 0.f;
+        const int cj = imax_d(__shfl(c, j), 0);
         rj[u] = part + (int64_t)cj * NQ * REC;
       }
       float xr[8][DPL];
@@ -435,7 +520,7 @@ __global__ __launch_bounds__(64) void decode_merge_kernel(const DecodeArgs a) {
 #pragma unroll
         for (int i = 0; i < DPL; ++i) {
           const int dd = lane + 64 * i;
-          xr[u][i] = dd < D ? rj[u][dd] : 0.f;
+          xr[u][i] = inside(dd) && on[u] ? rj[u][dd] : 0.f;
         }
 #pragma unroll
       for (int u = 0; u < 8; ++u)
@@ -446,24 +531,23 @@ __global__ __launch_bounds__(64) void decode_merge_kernel(const DecodeArgs a) {
   {
     const float f0 = c0 >= 0 ? fast_exp2(m0 - mu) : 0.f;
     L += c0 >= 0 ? f0 * l0 : 0.f;
-    const int nk = imin_d(64, total);
 #pragma unroll
     for (int u = 0; u < kMergeAhead; ++u) {
       const float fu = __shfl(f0, u);
-      if (u < nk) {
+      if (u < nk && ((live_lanes >> u) & 1)) {
 #pragma unroll
         for (int i = 0; i < DPL; ++i) A[i] = fmaf(fu, x[u][i], A[i]);
       }
     }
-    accumulate(c0, f0, kMergeAhead, nk);
+    accumulate(c0, f0, kMergeAhead, nk, live_lanes);
   }
-  for (int k0 = 64; k0 < total; k0 += 64) {
+  for (int k0 = 64; !DIRECT && k0 < total; k0 += 64) {
     const int c = k0 + lane < total ? live_chunk(a, nc, k0 + lane) : -1;
     const float* rec = part + (int64_t)(c < 0 ? 0 : c) * NQ * REC;
     const float mrec = rec[D], lrec = rec[D + 1];  // chunk 0's record for idle lanes: in bounds
     const float f = c >= 0 ? fast_exp2(mrec - mu) : 0.f;
     L += c >= 0 ? f * lrec : 0.f;
-    accumulate(c, f, 0, imin_d(64, total - k0));
+    accumulate(c, f, 0, imin_d(64, total - k0), ~0ull);
   }
   L = xor_sum<64>(L);
 #pragma unroll
@@ -472,34 +556,36 @@ __global__ __launch_bounds__(64) void decode_merge_kernel(const DecodeArgs a) {
     const float f = fast_exp2(es[e] - mu);
     L += f;
 #pragma unroll
-    for (int i = 0; i < DPL; ++i) A[i] = fmaf(f, evd[e][i], A[i]);
+    for (int i = 0; i < DPL; ++i) A[i] = fmaf(f, raw_as_f32(evd[e][i], a.e_dtype), A[i]);
   }
   const float inv = L > 0.f ? 1.f / L : 0.f;
   float* orow = a.out + b * a.o_sb + qi * a.o_ss + h * a.o_sh;
 #pragma unroll
   for (int i = 0; i < DPL; ++i) {
     const int dd = lane + 64 * i;
-    if (dd < D) orow[dd] = A[i] * inv;
+    if (inside(dd)) orow[dd] = A[i] * inv;
   }
 
   // The folded KV update of this (sequence, head), as sps_kv_update does it, from the old lengths.
-  if (upd && snap[kSnapActive] != 0) {
+  if (upd && snap_word(kSnapActive) != 0) {
     const KvUpdateArgs& u = a.upd;
-    const int64_t rlen = snap[kSnapRingLen], rpos = snap[kSnapRingPos], tlen = snap[kSnapRetLen];
+    const int64_t rlen = snap_word(kSnapRingLen), rpos = snap_word(kSnapRingPos), tlen = snap_word(kSnapRetLen);
     const int64_t slot = rlen >= u.window ? rpos : rlen;
     const bool ring_write = u.window > 0 && slot >= 0 && slot < u.ring_storage;
     const bool ret_write = tlen >= 0 && tlen < u.ret_storage;
     const int esz = u.kv_dtype == 2 ? 4 : 2;
+    auto row = [&](void* p, int64_t sb, int64_t sh, int64_t st, int64_t t) {
+      return scalar(static_cast<char*>(p) + (b * sb + h * sh + t * st) * esz);
+    };
+    char* const rk = row(u.ring_k, u.rk_sb, u.rk_sh, u.rk_st, slot);
+    char* const rv = row(u.ring_v, u.rv_sb, u.rv_sh, u.rv_st, slot);
+    char* const tk = row(u.ret_k, u.tk_sb, u.tk_sh, u.tk_st, tlen);
+    char* const tv = row(u.ret_v, u.tv_sb, u.tv_sh, u.tv_st, tlen);
 #pragma unroll
     for (int i = 0; i < kUpdPieces; ++i) {
-      const int pc = lane + 64 * i, r = pc / upr, j = pc - r * upr;
+      const int pc = lane + 64 * i, r = pc >> upr_shift, j = pc - (r << upr_shift);
       if (r >= 4 || !(r < 2 ? ring_write : ret_write)) continue;
-      void* dst = r == 0 ? u.ring_k : r == 1 ? u.ring_v : r == 2 ? u.ret_k : u.ret_v;
-      const int64_t db = r == 0 ? u.rk_sb : r == 1 ? u.rv_sb : r == 2 ? u.tk_sb : u.tv_sb;
-      const int64_t dh = r == 0 ? u.rk_sh : r == 1 ? u.rv_sh : r == 2 ? u.tk_sh : u.tv_sh;
-      const int64_t dt = r == 0 ? u.rk_st : r == 1 ? u.rv_st : r == 2 ? u.tk_st : u.tv_st;
-      const int64_t t = r < 2 ? slot : tlen;
-      *reinterpret_cast<u32x4_t*>(static_cast<char*>(dst) + (b * db + h * dh + t * dt) * esz + j * 16) = uval[i];
+      *reinterpret_cast<u32x4_t*>((r == 0 ? rk : r == 1 ? rv : r == 2 ? tk : tv) + j * 16) = uval[i];
     }
     if (lane == 0) {
       if (ret_write) cache_len_store(u.ret_len, b * u.ret_len_sb + h * u.ret_len_sh, u.len_i64, tlen + 1);
@@ -513,22 +599,47 @@ __global__ __launch_bounds__(64) void decode_merge_kernel(const DecodeArgs a) {
   }
 }
 
+template <int D, int NQ>
+static hipError_t launch_merge(const DecodeArgs& a, hipStream_t stream) {
+  const dim3 grid(NQ, a.H, a.B), block(64);
+  auto launch = [&](auto width_tag) {
+    constexpr int W = decltype(width_tag)::value;
+    if (a.n_chunks <= 64)
+      hipLaunchKernelGGL((decode_merge_kernel<D, NQ, true, W>), grid, block, 0, stream, a);
+    else
+      hipLaunchKernelGGL((decode_merge_kernel<D, NQ, false, W>), grid, block, 0, stream, a);
+  };
+  const bool q32 = a.q_dtype == 2, e32 = a.n_extra > 0 ? a.e_dtype == 2 : q32;
+  if (q32 != e32)
+    launch(std::integral_constant<int, 0>{});
+  else if (q32)
+    launch(std::integral_constant<int, 4>{});
+  else
+    launch(std::integral_constant<int, 2>{});
+  return hipGetLastError();
+}
+
 template <int D, int NQ, class KV>
 static hipError_t launch_decode_t(const DecodeArgs& a, hipStream_t stream) {
   if (a.B == 0 || a.H == 0) return hipSuccess;
   if (a.n_chunks > 0) {
     constexpr bool k16 = sizeof(typename KV::raw) == 2;
+    const dim3 grid(a.n_chunks, a.H, a.B);
+    auto launch = [&](auto pq_tag) {
+      constexpr bool PQ = decltype(pq_tag)::value;
+      if (a.pass == 8)
+        hipLaunchKernelGGL((decode_partial_kernel<D, NQ, KV, PQ, 8>), grid, dim3(256), 0, stream, a);
+      else
+        hipLaunchKernelGGL((decode_partial_kernel<D, NQ, KV, PQ, 16>), grid, dim3(256), 0, stream, a);
+    };
     if (k16 && a.q_packed)
-      hipLaunchKernelGGL((decode_partial_kernel<D, NQ, KV, k16>), dim3(a.n_chunks, a.H, a.B), dim3(256), 0,
-                         stream, a);
+      launch(std::integral_constant<bool, k16>{});
     else
-      hipLaunchKernelGGL((decode_partial_kernel<D, NQ, KV, false>), dim3(a.n_chunks, a.H, a.B), dim3(256), 0,
-                         stream, a);
+      launch(std::false_type{});
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
   }
-  hipLaunchKernelGGL((decode_merge_kernel<D, NQ>), dim3(NQ, a.H, a.B), dim3(64), 0, stream, a);
-  return hipGetLastError();
+  return launch_merge<D, NQ>(a, stream);
 }
 
 template <int D, int NQ>

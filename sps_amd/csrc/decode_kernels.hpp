@@ -8,21 +8,32 @@ namespace sps {
 constexpr int kMaxDecodeSegs = 3;
 constexpr int kMaxDecodeExtras = 2;
 
-// Work geometry for head dim D and K/V element size (bytes): each lane issues PASS 16-byte loads
+// Work geometry for head dim D, K/V element size (bytes) and PASS: each lane issues PASS 16-byte loads
 // of K and of V; a workgroup of 4 waves covers CHUNK keys of one segment.
-template <int D, int BYTES>
+template <int D, int BYTES, int PASS>
 struct DecodeGeom {
   static constexpr int EPL = 16 / BYTES;
   static constexpr int LPR = D / EPL;
   static constexpr int RPP = 64 / LPR;
-  static constexpr int PASS = 16;
   static constexpr int CHUNK = 4 * RPP * PASS;
-  static constexpr int REC = D + 4;  // floats per partial record: acc[D], m, l, 2 pad
 };
 
-// Host-side helper with the same numbers (the kernels static_assert agreement).
-inline int decode_chunk_keys(int D, int kv_bytes) { return 4 * (64 / (D / (16 / kv_bytes))) * 16; }
-inline int decode_record_floats(int D) { return D + 4; }
+// Loads per lane of a launch, from the sizes the host knows. 16 (512 keys a chunk at D = 64 in 16 bits)
+// where the grid has work to spare; 8 where all chunks of 16 loads would be at most 2048 workgroups
+// (8 per CU): there half the chunk fills the last wave of workgroups better (MI355X, q = 2, D = 64,
+// partial kernel: 16 sequences x 12 heads of ~2500 keys 30.1 -> 28.1 us, one sequence 10.5 -> 9.1 us),
+// while with more workgroups the merge pays for the extra records (64 x 16 of ~2300 keys, q = 1:
+// partial unchanged, merge +0.7 us). 2048 workgroups also bound the records to 8.5 MB.
+constexpr int kDecodeSmallGrid = 2048;
+inline int decode_pass(int B, int H, int D, int kv_bytes, int n_seg, const int64_t* scan) {
+  const int coarse = 4 * (64 / (D / (16 / kv_bytes))) * 16;
+  int64_t chunks = 0;
+  for (int s = 0; s < n_seg; ++s) chunks += (scan[s] + coarse - 1) / coarse;
+  return (int64_t)B * H * chunks <= kDecodeSmallGrid ? 8 : 16;
+}
+inline int decode_chunk_keys(int D, int kv_bytes, int pass) { return 4 * (64 / (D / (16 / kv_bytes))) * pass; }
+// Floats per partial record: acc[D], m, l, 2 pad.
+constexpr int decode_record_floats(int D) { return D + 4; }
 
 // Decode KV-cache update of one layer: ring (normal window) insert + retained append.
 constexpr int kMaxVecHeads = 1024;  // heads per sequence the 16-byte path keeps in LDS
@@ -86,7 +97,8 @@ struct DecodeArgs {
   float scale2;                 // sm_scale * log2(e)
   float* part;                  // workspace: [B*H, n_chunks, NQ, REC] partials
   int n_chunks;
-  int chunk_keys;
+  int chunk_keys, chunk_shift;  // a power of two and its logarithm
+  int pass;  // decode_pass()
   float* out;  // fp32, strides (b, slot, h), d stride 1
   int64_t o_sb, o_ss, o_sh;
   // KV update folded into the launch (sps_decode_kv_update), when snap is not null: the partial
@@ -108,6 +120,12 @@ __device__ __forceinline__ float load_as_f32(const void* p, int64_t i, int dtype
   const uint16_t x = reinterpret_cast<const uint16_t*>(p)[i];
   if (dtype == 1) return (float)__builtin_bit_cast(_Float16, x);
   return __builtin_bit_cast(float, (uint32_t)x << 16);
+}
+
+// The fp32 value of the raw bits (16 bits in the low half, or 32) of a bf16 / f16 / f32 element.
+__device__ __forceinline__ float raw_as_f32(uint32_t x, int dtype) {
+  const float h = (float)__builtin_bit_cast(_Float16, (uint16_t)(x & 0xffffu));
+  return dtype == 1 ? h : __builtin_bit_cast(float, dtype == 2 ? x : x << 16);
 }
 
 // Lengths and positions (int32 or int64) and active flags (1, 4 or 8 bytes) of the KV caches.
