@@ -11,14 +11,14 @@
 // from the run bounds, in closed form from the tile's first and last rows) in decreasing order of block count, so the heaviest workgroups are
 // dispatched first and each workgroup starts its first tile loads after reading one plan. The order
 // only affects speed: it is always a permutation of the tiles.
+#include <type_traits>
+
 #include "attn_kernels.hpp"
 
 namespace sps {
 
 constexpr int kPrepThreads = 1024;
-constexpr int kRegIds = 8;  // ids per thread held in registers (rows up to kPrepThreads * kRegIds positions)
 constexpr int kMaxSortTiles = 2048;  // rows with more tiles keep the closed-form order
-constexpr int kLdsRow = kPrepThreads * kRegIds;  // rows up to this length keep their runs in LDS
 
 // Exclusive scans of the per-thread chunk summaries, both in one pass so their latencies overlap:
 // a max-scan of `up` in thread order and a min-scan of `down` in reverse thread order. Inside each
@@ -115,35 +115,54 @@ __device__ void sort_tiles(const int* cost, int n, int first, int count, Emit em
   }
 }
 
+// One workgroup a row: bound by the instructions and latencies of its phases on one CU, not by bytes.
+// kRegIds is therefore no larger than the row needs (MI355X: N = 2048 with 8 ids a thread 7.0-8.1 us,
+// with 2 5.0-6.2; N = 4096 with 8 9.5, with 4 8.0).
+// kRegIds: ids per thread held in registers; rows of up to kPrepThreads * kRegIds positions keep their
+// ids there and their runs in LDS.
+template <int kRegIds>
 __global__ __launch_bounds__(kPrepThreads) void row_layout_kernel(const AttnArgs a) {
+  constexpr int kLdsRow = kPrepThreads * kRegIds;
   __shared__ __attribute__((aligned(16))) int s_scan[kPrepThreads];
   __shared__ int s_cost[kMaxSortTiles], s_cost_k[kMaxSortTiles];
   __shared__ int s_qplan[kMaxSortTiles][4], s_kplan[kMaxSortTiles][2];
   __shared__ int s_nonmono;
-  __shared__ short s_start[kLdsRow], s_end[kLdsRow];
+  __shared__ __attribute__((aligned(16))) uint16_t s_start[kLdsRow], s_end[kLdsRow];
   const MaskSpec m = a.m;
   const int b = blockIdx.x, tid = threadIdx.x, N = m.N;
   int* start = a.run_start + (int64_t)b * N;
   int* end = a.run_end + (int64_t)b * N;
-  const int C = (N + kPrepThreads - 1) / kPrepThreads;
+  // Rows that fit give each thread kRegIds consecutive positions, longer ones an even share.
+  const bool in_regs = N <= kLdsRow;
+  const int C = in_regs ? kRegIds : (N + kPrepThreads - 1) / kPrepThreads;
   const int p0 = imin(tid * C, N), p1 = imin(p0 + C, N);
   if (tid == 0) s_nonmono = 0;
 
-  const bool in_regs = C <= kRegIds;
   int last = -1, first = N;
   bool dec = false;
   int64_t d[kRegIds];
   bool flag[kRegIds];
   if (in_regs) {
-    // Common case: every id of this thread's chunk (and its predecessor) loaded once, together: one
-    // branch on the id type around straight-line loads whose positions are clamped into the row
-    // (values past the chunk are never used), so all of them are in flight at once.
+    // Common case: every id of this thread's chunk (and its predecessor) loaded once, together, in
+    // 16-byte pieces where the row is aligned and the chunk whole, else one by one with positions clamped
+    // into the row (values past the chunk are never used).
     int64_t before = 0;
     auto load_all = [&](auto* ids) {
+      using T = std::remove_cv_t<std::remove_pointer_t<decltype(ids)>>;
       ids += (int64_t)b * a.docs_sb;
+      constexpr int kBytes = kRegIds * (int)sizeof(T), kVec = kBytes < 16 ? kBytes : 16;
+      typedef T vec_t __attribute__((ext_vector_type(kVec / (int)sizeof(T))));
       const int64_t bv = ids[imax(imin(p0, N) - 1, 0)];
+      if ((reinterpret_cast<uintptr_t>(ids) & (kVec - 1)) == 0 && p0 + kRegIds <= N) {
+        vec_t x[kBytes / kVec];
 #pragma unroll
-      for (int j = 0; j < kRegIds; ++j) d[j] = ids[imin(p0 + j, N - 1)];
+        for (int v = 0; v < kBytes / kVec; ++v) x[v] = reinterpret_cast<const vec_t*>(ids + p0)[v];
+#pragma unroll
+        for (int j = 0; j < kRegIds; ++j) d[j] = x[j * (int)sizeof(T) / kVec][j % (kVec / (int)sizeof(T))];
+      } else {
+#pragma unroll
+        for (int j = 0; j < kRegIds; ++j) d[j] = ids[imin(p0 + j, N - 1)];
+      }
       before = (p0 > 0 && p0 < N) ? bv : 0;
     };
     if (a.docs_i64)
@@ -179,19 +198,25 @@ __global__ __launch_bounds__(kPrepThreads) void row_layout_kernel(const AttnArgs
   block_exclusive_scans(s_scan, s_scan + kPrepWaves, last, first, -1, N, carry_start, carry_next);
   const bool mono = s_nonmono == 0;
 
-  if (mono && in_regs) {
-    // LDS copies only; the global arrays are written from them below with coalesced stores.
-    int cur = carry_start;
+  int cs[kRegIds], ce[kRegIds];  // run bounds of the thread's positions (rows that fit)
+  if (in_regs) {
+    int cur = carry_start, nxt = carry_next;
 #pragma unroll
     for (int j = 0; j < kRegIds; ++j) {
       if (flag[j]) cur = p0 + j;
-      if (p0 + j < p1) s_start[p0 + j] = (short)cur;
+      cs[j] = mono ? cur : 0;
     }
-    int nxt = carry_next;
 #pragma unroll
     for (int j = kRegIds - 1; j >= 0; --j) {
-      if (p0 + j < p1) s_end[p0 + j] = (short)(nxt - 1);
+      ce[j] = mono ? nxt - 1 : N - 1;
       if (flag[j]) nxt = p0 + j;
+    }
+    // Into LDS for the plans, two positions a word (a partial chunk's rest lies inside the arrays); the
+    // global arrays follow once the plans can start.
+#pragma unroll
+    for (int j = 0; j < kRegIds; j += 2) {
+      reinterpret_cast<uint32_t*>(s_start)[(tid * kRegIds + j) / 2] = (uint32_t)(cs[j] & 0xffff) | (uint32_t)cs[j + 1] << 16;
+      reinterpret_cast<uint32_t*>(s_end)[(tid * kRegIds + j) / 2] = (uint32_t)(ce[j] & 0xffff) | (uint32_t)ce[j + 1] << 16;
     }
   } else if (mono) {
     int cur = carry_start;
@@ -209,32 +234,42 @@ __global__ __launch_bounds__(kPrepThreads) void row_layout_kernel(const AttnArgs
     }
   } else {
     for (int p = p0; p < p1; ++p) {
-      if (in_regs) {
-        s_start[p] = 0;
-        s_end[p] = (short)(N - 1);
-      } else {
-        start[p] = 0;
-        end[p] = N - 1;
-      }
+      start[p] = 0;
+      end[p] = N - 1;
     }
   }
   if (tid == 0) a.row_mono[b] = mono ? 1 : 0;
-  __syncthreads();  // start/end of the whole row are visible to every thread below
   if (in_regs) {
-    // Rows held in LDS go to global memory now: one pass of consecutive positions per thread group,
-    // 4 per thread (16-byte stores) when the row length allows; the stores drain while the plans
-    // below are computed (the barrier before the sorts is the first to wait for them).
-    if ((N & 3) == 0) {
-      for (int p = 4 * tid; p < N; p += 4 * kPrepThreads) {
-        *reinterpret_cast<int4*>(start + p) = make_int4(s_start[p], s_start[p + 1], s_start[p + 2], s_start[p + 3]);
-        *reinterpret_cast<int4*>(end + p) = make_int4(s_end[p], s_end[p + 1], s_end[p + 2], s_end[p + 3]);
+    lds_barrier();  // the plans read only LDS
+    // The global arrays, 4 (2) positions a store where the rows are aligned; the stores drain while the
+    // plans below are computed.
+    constexpr int kStore = kRegIds < 4 ? kRegIds : 4;
+    typedef int store_t __attribute__((ext_vector_type(kStore)));
+    if ((N & (kStore - 1)) == 0) {
+      if (p0 < N) {
+#pragma unroll
+        for (int j = 0; j < kRegIds; j += kStore) {
+          if (p0 + j >= N) continue;
+          store_t vs, ve;
+#pragma unroll
+          for (int u = 0; u < kStore; ++u) {
+            vs[u] = cs[j + u];
+            ve[u] = ce[j + u];
+          }
+          *reinterpret_cast<store_t*>(start + p0 + j) = vs;
+          *reinterpret_cast<store_t*>(end + p0 + j) = ve;
+        }
       }
     } else {
-      for (int p = tid; p < N; p += kPrepThreads) {
-        start[p] = s_start[p];
-        end[p] = s_end[p];
+#pragma unroll
+      for (int j = 0; j < kRegIds; ++j) {
+        if (p0 + j >= N) continue;
+        start[p0 + j] = cs[j];
+        end[p0 + j] = ce[j];
       }
     }
+  } else {
+    __syncthreads();  // start/end of the whole row are visible to every thread below
   }
   // Rows that fit read their run bounds from LDS (short: positions < kLdsRow <= 32767).
   const bool lds_ok = in_regs;
@@ -320,7 +355,13 @@ __global__ __launch_bounds__(kPrepThreads) void row_layout_kernel(const AttnArgs
 
 hipError_t launch_row_layout(const AttnArgs& a, hipStream_t stream) {
   if (a.B == 0 || a.m.N == 0 || !a.m.has_docs) return hipSuccess;
-  hipLaunchKernelGGL(row_layout_kernel, dim3(a.B), dim3(kPrepThreads), 0, stream, a);
+  const dim3 grid(a.B), block(kPrepThreads);
+  if (a.m.N <= 2 * kPrepThreads)
+    hipLaunchKernelGGL(row_layout_kernel<2>, grid, block, 0, stream, a);
+  else if (a.m.N <= 4 * kPrepThreads)
+    hipLaunchKernelGGL(row_layout_kernel<4>, grid, block, 0, stream, a);
+  else
+    hipLaunchKernelGGL(row_layout_kernel<8>, grid, block, 0, stream, a);
   return hipGetLastError();
 }
 
