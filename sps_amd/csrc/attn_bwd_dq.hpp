@@ -24,7 +24,8 @@ constexpr int bwd_waves() { return D <= 64 ? 2 : 1; }
 // as many workgroups as the registers: three waves per SIMD at D = 64 (168 VGPRs; dQ -4 % at C3, -6 %
 // at C2 against four-block groups at 2 waves per SIMD), two at D = 128 (256 VGPRs, none spilled under
 // the default scheduler with two id checks in flight; against four-block groups at one wave per SIMD:
-// B2 H16 N4096 126 -> 119 us, f16 B3 H10 N3062 70 -> 64 us).
+// B2 H16 N4096 over several document layouts 122-126 -> 119-122 us and at best 95 -> 76 us, though one
+// layout of short documents 112 -> 119 us; f16 B3 H10 N3062 70 -> 64 us).
 template <int D>
 constexpr int dq_group() { return D == 64 || D == 128 ? 2 : bwd_group<D>(); }
 template <int D>
