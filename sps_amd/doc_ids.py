@@ -38,7 +38,8 @@ def document_ids(idx_BxT: Tensor, *, eos_token_id: int, pad_token_id: int, repea
     if out_dtype not in _INT_CODES:
         raise TypeError(f"document ids must be int32 or int64, got {out_dtype}")
     out = torch.empty((b, t * repeat), dtype=out_dtype, device=tok.device)
-    bad = torch.empty((b,), dtype=torch.int32, device=tok.device) if validate else None  # the kernel writes every flag
+    # The kernel writes every row's flag; rows without tokens launch none (and are left padded).
+    bad = torch.empty((b,), dtype=torch.int32, device=tok.device) if validate and t else None
     status = N.lib().sps_document_ids(
         b, t, tok.data_ptr(), _INT_CODES[tok.dtype], tok.stride(0) if b > 1 else t, int(eos_token_id),
         int(pad_token_id), int(repeat), out.data_ptr(), _INT_CODES[out_dtype], out.stride(0) if b > 1 else t * repeat,

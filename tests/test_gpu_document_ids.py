@@ -118,3 +118,16 @@ def test_ids_feed_the_attention_kernel():
     got = SA.attention_mask(N.FAMILY_SPS, 800, ids, window=16).cpu().numpy().astype(bool)
     want = M.batch_mask(N.FAMILY_SPS, docidx.interleave(docidx.document_idx(rows, EOS, PAD)), window=16)
     assert (got == want).all()
+
+
+@pytest.mark.parametrize("b,t", [(3, 0), (0, 0), (0, 5)])
+@pytest.mark.parametrize("repeat", [1, 2])
+def test_empty_rows(b, t, repeat):
+    # No kernel runs on empty rows, so nothing may be read from a buffer it would have filled: the
+    # allocator's small blocks are left holding non-zero values first.
+    tok = torch.empty((b, t), dtype=torch.int64, device="cuda")
+    dirty = [torch.full((128,), 1, dtype=torch.int32, device="cuda") for _ in range(64)]
+    del dirty
+    for _ in range(4):
+        ids = document_ids(tok, eos_token_id=EOS, pad_token_id=PAD, repeat=repeat)
+        assert ids.shape == (b, t * repeat) and ids.dtype == torch.int64
