@@ -154,6 +154,10 @@ AttnOut attn_forward(const Tensor& q, const Tensor& k, const Tensor& v, const Te
 }
 
 struct AttentionFunction : torch::autograd::Function<AttentionFunction> {
+  // Compiled autograd may trace the backward (its tensors are then not plain, so it goes through the
+  // registered op); otherwise each call would be a graph break, and an error with fullgraph.
+  static constexpr bool is_traceable = true;
+
   static Tensor forward(torch::autograd::AutogradContext* ctx, const Tensor& q, const Tensor& k, const Tensor& v,
                         const std::optional<Tensor>& docs_opt, double sm_scale, int64_t family, int64_t window,
                         bool has_pkw, int64_t pkw) {
@@ -307,6 +311,8 @@ std::vector<Tensor> rope_launch(const Tensor& q, const Tensor& k, const Tensor& 
 
 // v undefined: RoPE of a pair, outputs [B, N, H, D]; defined: outputs are [B, H, N, D] views.
 struct RopeFunction : torch::autograd::Function<RopeFunction> {
+  static constexpr bool is_traceable = true;  // as AttentionFunction's
+
   static torch::autograd::variable_list forward(torch::autograd::AutogradContext* ctx, const Tensor& q, const Tensor& k,
                                                 const std::optional<Tensor>& v_opt, const Tensor& freqs,
                                                 int64_t out_type) {

@@ -157,3 +157,50 @@ def test_inductor_compiled_block_matches_eager(monkeypatch):
         results.append([loss.detach()] + [p.grad.clone() for p in (*c_attn.parameters(), *c_proj.parameters())])
     for got, want in zip(results[1], results[0]):
         torch.testing.assert_close(got, want, atol=1e-4, rtol=2e-2)
+
+
+@pytest.mark.parametrize("docs", [False, True])
+@pytest.mark.parametrize("pair", [False, True])
+def test_compiled_autograd_of_an_eager_forward(docs, pair):
+    # An eager forward (the native autograd functions) whose backward compiled autograd captures as one
+    # graph: the functions' backward is traced through the registered ops.
+    torch._dynamo.reset()
+    g = torch.Generator().manual_seed(7)
+    b, n, h, d = 2, 128, 2, 32
+    base = [torch.randn((b, n, h, d), generator=g).cuda() for _ in range(3)]
+    freqs = torch.polar(torch.ones(n, d // 2), torch.randn((n, d // 2), generator=g)).cuda()
+    ids = torch.tensor([[0] * 50 + [1] * 78] * b, device="cuda") if docs else None
+
+    def loss_of(x):
+        if pair:
+            q, k = (t.to(torch.bfloat16).transpose(1, 2).contiguous() for t in sps_amd.apply_rotary_emb(x[0], x[1], freqs))
+            v = x[2].to(torch.bfloat16).transpose(1, 2).contiguous()
+        else:
+            q, k, v = sps_amd.rope_qkv_for_attention(*x, freqs)
+        o = sps_amd.sps_sliding_attention(q, k, v, d ** -0.5, 16, documents_idx_BxT=ids)
+        return (o.float() * torch.arange(n, device="cuda")[None, None, :, None]).sum()
+
+    grads = []
+    for compiled in (False, True):
+        x = [t.clone().requires_grad_() for t in base]
+        loss = loss_of(x)
+        assert "AttentionFunction" in str(_names(loss.grad_fn))  # the native forward, not the registered op
+        if compiled:
+            with torch._dynamo.compiled_autograd._enable(torch.compile(backend="aot_eager", fullgraph=True)):
+                loss.backward()
+        else:
+            loss.backward()
+        grads.append([t.grad for t in x])
+    for x, y in zip(*grads):
+        assert torch.equal(x, y)
+
+
+def _names(fn):
+    """The names of a graph's nodes."""
+    seen, todo = set(), [fn]
+    while todo:
+        node = todo.pop()
+        if node is not None and node not in seen:
+            seen.add(node)
+            todo += [f for f, _ in node.next_functions]
+    return {node.name() for node in seen}
