@@ -162,7 +162,13 @@ int sps_attn_mask(int family, int B, int N,
                   int window, int has_pkw, int pkw, int schedule, uint8_t* mask,
                   void* workspace, size_t workspace_bytes, void* stream);
 
-/* Workspace needed by sps_decode for the given segment scan lengths. */
+/*
+ * Workspace of sps_decode for the given segment scan lengths. A workspace of these bytes also serves
+ * every call with no longer scans, no larger B and no larger H (same D, nq and kv_dtype), so a caller
+ * may allocate it once for its largest call; where it holds too little for the smaller chunks that a
+ * small call would otherwise take, the call uses full ones (the sums' order is all that differs).
+ * sps_decode_kv_update_workspace_bytes behaves alike.
+ */
 size_t sps_decode_workspace_bytes(int B, int H, int D, int nq, int kv_dtype, int n_seg,
                                   const int64_t* seg_scan);
 

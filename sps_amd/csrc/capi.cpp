@@ -306,14 +306,18 @@ static int kv_bytes(int kv_dtype) { return kv_dtype == SPS_DTYPE_F32 ? 4 : 2; }
 
 static bool decode_head_dim(int D) { return D == 16 || D == 32 || D == 64 || D == 128 || D == 256; }
 
+// Bytes of the partial records of a decode in chunks of `pass` loads a lane.
+static size_t decode_part_bytes(int B, int H, int D, int nq, int kb, int n_seg, const int64_t* seg_scan, int pass) {
+  const int ck = sps::decode_chunk_keys(D, kb, pass);
+  int64_t chunks = 0;
+  for (int s = 0; s < n_seg; ++s) chunks += (seg_scan[s] + ck - 1) / ck;
+  return align_up((size_t)B * H * chunks * nq * sps::decode_record_floats(D) * sizeof(float));
+}
+
 size_t sps_decode_workspace_bytes(int B, int H, int D, int nq, int kv_dtype, int n_seg, const int64_t* seg_scan) {
   if (!decode_head_dim(D) || B < 0 || H < 0 || n_seg < 0 || n_seg > sps::kMaxDecodeSegs) return 0;
   const int kb = kv_bytes(kv_dtype);
-  const int ck = sps::decode_chunk_keys(D, kb, sps::decode_pass(B, H, D, kb, n_seg, seg_scan));
-  int64_t chunks = 0;
-  for (int s = 0; s < n_seg; ++s) chunks += (seg_scan[s] + ck - 1) / ck;
-  const size_t bytes = (size_t)B * H * chunks * nq * sps::decode_record_floats(D) * sizeof(float);
-  return align_up(bytes);
+  return decode_part_bytes(B, H, D, nq, kb, n_seg, seg_scan, sps::decode_pass(B, H, D, kb, n_seg, seg_scan));
 }
 
 }  // extern "C"
@@ -349,8 +353,17 @@ static int decode_impl(int B, int H, int D, int nq, const void* q, int q_dtype, 
   if ((int64_t)B * H == 0) return SPS_OK;
   if (!q || !q_strides || !out || !out_strides) return fail(SPS_E_INVALID, "q/out: null pointer");
   if (!(std::isfinite(sm_scale))) return fail(SPS_E_INVALID, "sm_scale must be finite");
-  const size_t part_bytes = sps_decode_workspace_bytes(B, H, D, nq, kv_dtype, n_seg, seg_scan);
-  const size_t need = part_bytes + (upd ? decode_snapshot_bytes(B, H) : 0);
+  const int kb = kv_bytes(kv_dtype);
+  const size_t snap_bytes = upd ? decode_snapshot_bytes(B, H) : 0;
+  int pass = sps::decode_pass(B, H, D, kb, n_seg, seg_scan);
+  size_t part_bytes = decode_part_bytes(B, H, D, nq, kb, n_seg, seg_scan, pass);
+  if (pass < 16 && workspace_bytes < part_bytes + snap_bytes) {
+    // The full chunks' records: no more than any larger call's workspace holds, so a workspace allocated
+    // once for the largest scan lengths, B and H serves every smaller call, whichever chunks it would take.
+    pass = 16;
+    part_bytes = decode_part_bytes(B, H, D, nq, kb, n_seg, seg_scan, pass);
+  }
+  const size_t need = part_bytes + snap_bytes;
   if (workspace_bytes < need) return fail(SPS_E_WORKSPACE, "workspace too small: %zu < %zu", workspace_bytes, need);
   sps::DecodeArgs a;
   std::memset(&a, 0, sizeof(a));
@@ -359,9 +372,7 @@ static int decode_impl(int B, int H, int D, int nq, const void* q, int q_dtype, 
   a.NQ = nq;
   a.n_seg = n_seg;
   a.n_extra = n_extra;
-  const int kb = kv_bytes(kv_dtype);
   const int epl = 16 / kb;
-  const int pass = sps::decode_pass(B, H, D, kb, n_seg, seg_scan);
   const int ck = sps::decode_chunk_keys(D, kb, pass);
   int chunk = 0;
   for (int s = 0; s < n_seg; ++s) {

@@ -59,3 +59,15 @@ def test_types_and_segments(d, kv, q_dtype, e_dtype):
         # Three segments (q = 1) over few chunks, and enough keys for more than 64 of them at D = 256.
         _check(2, 3, d, nq, kv, q_dtype, e_dtype, [33, 700, 64] if nq == 1 else [40, 2300], 2, d + nq)
     _check(2, 2, d, 1, kv, q_dtype, e_dtype, [90], 0, d)
+
+
+@pytest.mark.parametrize("nq", [1, 2])
+def test_workspace_of_a_larger_call(nq, monkeypatch):
+    # A workspace sized for 2049 workgroups of full chunks, then a call of half as many, which would take
+    # half-size chunks if the workspace held their records.
+    b, h, storage = 3, 683, 300
+    need = DA._decode_ws_bytes(False, b, h, 64, nq, 0, (storage,))
+    small = DA._decode_ws_bytes(False, b, 512, 64, nq, 0, (storage,))
+    assert need < small
+    monkeypatch.setattr(DA, "_decode_ws_bytes", lambda *a: need)
+    _check(b, 512, 64, nq, torch.bfloat16, torch.bfloat16, torch.bfloat16, [storage], 1, 3)

@@ -111,6 +111,39 @@ def test_decode_argument_validation():
     assert _decode(n_extra=1, extra_dtype=N.DTYPE_I64) == N.SPS_E_UNSUPPORTED and "extra" in N.last_error()
 
 
+@cpu_only
+@pytest.mark.parametrize("update", [False, True])
+@pytest.mark.parametrize("D,kv", [(16, N.DTYPE_BF16), (64, N.DTYPE_BF16), (64, N.DTYPE_F32), (128, N.DTYPE_F16),
+                                  (256, N.DTYPE_F32)])
+def test_decode_workspace_serves_smaller_calls(D, kv, update):
+    # A workspace sized for the largest scan lengths, batch and head count is enough for every smaller call,
+    # on both sides of the grid limits that pick the chunk size. The segments' pointers are null, so an
+    # accepted workspace ends in SPS_E_INVALID and nothing is launched.
+    lib, z, p = N.lib(), N.i64_array([0] * 8), 0x10000
+    size = lib.sps_decode_kv_update_workspace_bytes if update else lib.sps_decode_workspace_bytes
+    null, zi = N.ptr_const((0, 0)), N.i32_const((0, 0))
+
+    def call(b, h, nq, scans, ws_bytes):
+        head = (b, h, D, nq, p, N.DTYPE_BF16, z, kv, len(scans), null, z, null, z, null, zi, zi, N.i64_array(scans), 0,
+                None, None, N.DTYPE_BF16, z, None, 0.125, p, z)
+        if not update:
+            return lib.sps_decode(*head, p, ws_bytes, None)
+        return lib.sps_decode_kv_update(*head, p, p, z, 4, 2, p, p, z, p, p, z, 8, p, z, N.DTYPE_I64, kv, p, p, p, p, z,
+                                        p, N.DTYPE_U8, 1, p, ws_bytes, None)
+
+    keys = 4 * (64 // (D // (4 if kv == N.DTYPE_F32 else 8))) * 16  # a full chunk
+    scans = sorted({max(1, keys * c // 4 + e) for c in (1, 2, 4, 8, 15, 16, 31, 32, 33, 40, 48, 64, 128, 200) for e in (0, 1)})
+    for nq in (1, 2):
+        for b, h in ((1, 4), (16, 12), (21, 12), (22, 12), (64, 16)):
+            for longest in scans[::3]:
+                ws = size(b, h, D, nq, kv, 2, N.i64_array([64, longest]))
+                for b2 in sorted({1, b // 2, b - 1, b} - {0}):
+                    for scan in (s for s in scans if s <= longest):
+                        rc = call(b2, h, nq, (64, scan), ws)
+                        assert rc == N.SPS_E_INVALID and "null pointer" in N.last_error(), (b, h, longest, b2, scan)
+                assert call(b, h, nq, (64, longest), 0) == N.SPS_E_WORKSPACE
+
+
 def test_last_error_truncates():
     _fwd(family=9)
     buf = C.create_string_buffer(8)
