@@ -329,12 +329,9 @@ __device__ __forceinline__ float wave_max_f(float x) {
 // lengths. Chunks past those loaded ahead are read 8 records per batch once the max is known. WIDTH:
 // bytes per element of the query and the extras (0: they differ; the branch on the type then waits
 // for the loads before it).
-template <int D>
-constexpr int merge_ahead() { return D <= 128 ? 24 : 16; }
-
 template <int D, int NQ, bool DIRECT, int WIDTH>
 __global__ __launch_bounds__(64) void decode_merge_kernel(const DecodeArgs a) {
-  constexpr int kMergeAhead = merge_ahead<D>();
+  constexpr int kMergeAhead = decode_merge_ahead(D);
   constexpr int DPL = (D + 63) / 64;  // output elements per lane
   constexpr int REC = decode_record_floats(D);
   auto inside = [](int dd) { return D % 64 == 0 || dd < D; };  // lanes past D have no element

@@ -18,18 +18,32 @@ struct DecodeGeom {
   static constexpr int CHUNK = 4 * RPP * PASS;
 };
 
-// Loads per lane of a launch, from the sizes the host knows. 16 (512 keys a chunk at D = 64 in 16 bits)
-// where the grid has work to spare; 8 where all chunks of 16 loads would be at most 2048 workgroups
-// (8 per CU): there half the chunk fills the last wave of workgroups better (MI355X, q = 2, D = 64,
-// partial kernel: 16 sequences x 12 heads of ~2500 keys 30.1 -> 28.1 us, one sequence 10.5 -> 9.1 us),
-// while with more workgroups the merge pays for the extra records (64 x 16 of ~2300 keys, q = 1:
-// partial unchanged, merge +0.7 us). 2048 workgroups also bound the records to 8.5 MB.
+// Chunks whose records the merge loads ahead, before it knows the maximum.
+constexpr int decode_merge_ahead(int D) { return D <= 128 ? 24 : 16; }
+
+// Loads per lane of a launch, from the sizes the host knows: 16 (512 keys a chunk at D = 64 in 16 bits), or 8
+// where half the chunk pays (MI355X, D = 64, 16 bits, partial and merge, chunks of 16 against 8 loads).
+//  - The grid is small: at most 2048 workgroups of 16 loads (8 per CU). There half the chunk fills the last
+//    wave of workgroups better (q = 2, 16 sequences x 12 heads of ~2500 keys, partial 30.1 -> 28.1 us; one
+//    sequence 10.5 -> 9.1 us); with more the merge pays for the extra records (64 x 16 of ~2300 keys, q = 1:
+//    partial unchanged, merge +0.7 us). 2048 workgroups also bound the records to 8.5 MB.
+//  - The merge of a row is short: it walks the records past decode_merge_ahead one batch of 8 after another, and
+//    half the chunk doubles them (12 heads of one sequence: 1024 keys 10.3 -> 9.3 us, but 32768 keys
+//    22.5 -> 27.3 us; 2 heads of 262144 keys 44 -> 68 us; D = 128 in fp32, 8 heads of 8192 keys 13.0 -> 16.4 us).
+//    So all records lie among those loaded ahead, or, where the half chunks all run at once, one on a CU, within
+//    two more batches (33 of 4 heads, 12.1 -> 10.8 us; 41 of them 12.5 -> 13.0 us; 33 or more on more CUs than
+//    there are -5 to +9 %). At D = 256 a batch takes twice as long, so one more (25 half chunks: +2 to +19 %).
 constexpr int kDecodeSmallGrid = 2048;
 inline int decode_pass(int B, int H, int D, int kv_bytes, int n_seg, const int64_t* scan) {
-  const int coarse = 4 * (64 / (D / (16 / kv_bytes))) * 16;
-  int64_t chunks = 0;
-  for (int s = 0; s < n_seg; ++s) chunks += (scan[s] + coarse - 1) / coarse;
-  return (int64_t)B * H * chunks <= kDecodeSmallGrid ? 8 : 16;
+  const int64_t coarse = 4 * (64 / (D / (16 / kv_bytes))) * 16, fine = coarse / 2;
+  int64_t c = 0, f = 0;
+  for (int s = 0; s < n_seg; ++s) {
+    c += (scan[s] + coarse - 1) / coarse;
+    f += (scan[s] + fine - 1) / fine;
+  }
+  const int64_t rows = (int64_t)B * H;
+  const int more = rows * f <= 256 ? (D <= 128 ? 16 : 8) : 0;
+  return rows * c <= kDecodeSmallGrid && f <= decode_merge_ahead(D) + more ? 8 : 16;
 }
 inline int decode_chunk_keys(int D, int kv_bytes, int pass) { return 4 * (64 / (D / (16 / kv_bytes))) * pass; }
 // Floats per partial record: acc[D], m, l, 2 pad.

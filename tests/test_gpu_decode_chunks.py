@@ -61,6 +61,16 @@ def test_types_and_segments(d, kv, q_dtype, e_dtype):
     _check(2, 2, d, 1, kv, q_dtype, e_dtype, [90], 0, d)
 
 
+# The rows that end the half-size chunks: as many as the merge loads ahead (24; 16 at D = 256) and one more,
+# on a grid of one workgroup per CU and a larger one, and two batches of 8 past them (one at D = 256).
+@pytest.mark.parametrize("d,b,h,storage", [(64, 2, 8, 256 * 24), (64, 2, 8, 256 * 24 + 1), (64, 1, 2, 256 * 40),
+                                           (64, 1, 2, 256 * 40 + 1), (256, 2, 16, 64 * 16), (256, 2, 16, 64 * 16 + 1),
+                                           (256, 1, 3, 64 * 24), (256, 1, 3, 64 * 24 + 1)])
+@pytest.mark.parametrize("nq", [1, 2])
+def test_rows_at_the_merge_limits(d, b, h, storage, nq):
+    _check(b, h, d, nq, torch.bfloat16, torch.bfloat16, torch.bfloat16, [storage], 2 if nq == 2 else 1, storage)
+
+
 @pytest.mark.parametrize("nq", [1, 2])
 def test_workspace_of_a_larger_call(nq, monkeypatch):
     # A workspace sized for 2049 workgroups of full chunks, then a call of half as many, which would take

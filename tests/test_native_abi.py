@@ -111,6 +111,22 @@ def test_decode_argument_validation():
     assert _decode(n_extra=1, extra_dtype=N.DTYPE_I64) == N.SPS_E_UNSUPPORTED and "extra" in N.last_error()
 
 
+@pytest.mark.parametrize("D,kv", [(16, N.DTYPE_BF16), (64, N.DTYPE_BF16), (128, N.DTYPE_F32), (256, N.DTYPE_F16)])
+def test_decode_chunks_of_long_rows(D, kv):
+    # A row whose records the merge cannot load ahead keeps full chunks however small the grid is: half-size
+    # ones would double the records it walks. Read off the workspace, which holds the records.
+    lib = N.lib()
+    keys = 4 * (64 // (D // (4 if kv == N.DTYPE_F32 else 8))) * 16  # a full chunk
+    rec = (D + 4) * 4
+    ahead, more = (24, 16) if D <= 128 else (16, 8)
+    up = lambda x: (x + 255) // 256 * 256  # noqa: E731
+    for b, h in ((1, 1), (1, 4), (2, 8), (8, 16)):
+        for chunks in (1, 4, ahead // 2, ahead // 2 + 1, (ahead + more) // 2, (ahead + more) // 2 + 1, 64, 300):
+            got = lib.sps_decode_workspace_bytes(b, h, D, 1, kv, 1, N.i64_array([chunks * keys]))
+            half = 2 * chunks <= ahead + (more if b * h * 2 * chunks <= 256 else 0) and b * h * chunks <= 2048
+            assert got == up(b * h * chunks * (2 if half else 1) * rec), (b, h, chunks)
+
+
 @cpu_only
 @pytest.mark.parametrize("update", [False, True])
 @pytest.mark.parametrize("D,kv", [(16, N.DTYPE_BF16), (64, N.DTYPE_BF16), (64, N.DTYPE_F32), (128, N.DTYPE_F16),
