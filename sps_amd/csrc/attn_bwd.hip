@@ -401,14 +401,13 @@ static hipError_t launch_bwd_t(const AttnArgs& a, int passes, hipStream_t stream
   const int64_t nq = (int64_t)q_tiles(a.m.N) * a.B * a.H;
   const int64_t nk = (int64_t)k_tiles(a.m.family, a.m.N, a.m.P) * a.B * a.H;
   if ((passes & kBwdDq) && nq > 0) {
-    if constexpr (D == 128) {
-      const hipError_t e = launch_attn_bwd_dq_128(a, std::is_same<E, ElemF16>::value, nq, stream);
-      if (e != hipSuccess) return e;
-    } else {
-      hipLaunchKernelGGL((attn_bwd_dq_kernel<D, E>), dim3((unsigned)nq), dim3(256), 0, stream, a);
-      const hipError_t e = hipGetLastError();
-      if (e != hipSuccess) return e;
-    }
+    const dim3 grid((unsigned)nq), block(256);
+    if (D == 128 && dq_two_waves(a.m, nq))
+      hipLaunchKernelGGL((attn_bwd_dq_kernel<D, E, D == 128 ? 2 : dq_waves<D>()>), grid, block, 0, stream, a);
+    else
+      hipLaunchKernelGGL((attn_bwd_dq_kernel<D, E>), grid, block, 0, stream, a);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
   }
   if ((passes & kBwdDkdv) && nk > 0) {
     // From D = 128 on a wave cannot hold K, V, dK and dV of 32 keys beside another wave: two share them.

@@ -1,6 +1,4 @@
-// The dQ pass of the backward attention (see attn_bwd.hip for the two passes). Head dim 128 is
-// instantiated in attn_bwd_split.hip, whose scheduling leaves it two waves per SIMD without spills, the
-// others in attn_bwd.hip.
+// The dQ pass of the backward attention (see attn_bwd.hip for the two passes).
 #pragma once
 #include "attn_tiles.hpp"
 
@@ -22,14 +20,17 @@ constexpr int bwd_waves() { return D <= 64 ? 2 : 1; }
 
 // The dQ pass in groups of two blocks (32 KiB of tiles at D = 64, 64 KiB at D = 128), so the LDS holds
 // as many workgroups as the registers: three waves per SIMD at D = 64 (168 VGPRs; dQ -4 % at C3, -6 %
-// at C2 against four-block groups at 2 waves per SIMD), two at D = 128 (256 VGPRs, none spilled under
-// the default scheduler with two id checks in flight; against four-block groups at one wave per SIMD:
-// B2 H16 N4096 over several document layouts 122-126 -> 119-122 us and at best 95 -> 76 us, though one
-// layout of short documents 112 -> 119 us; f16 B3 H10 N3062 70 -> 64 us).
+// at C2 against four-block groups at 2 waves per SIMD). D = 128 has two forms, picked by dq_two_waves():
+// four-block groups at one wave per SIMD (345 VGPRs), and two-block groups at two (256 VGPRs, 28 spilled). Both
+// need the iterative ILP schedule of attn_bwd.hip, spills and all: under the default scheduler the two-wave form
+// spills none, but a workgroup that ends up alone on its CU then takes ~30 % longer than the one-wave form, which
+// small grids and layouts with one long document are made of (MI355X, dQ, one wave / two waves with ILP
+// / two without: C4 118.5 / 107.2 / 120.3 us, B2 H16 N2048 dense causal 72.7 / 69.9 / 78.0, B4 H16 N4096
+// 227 / 190 / 191).
 template <int D>
-constexpr int dq_group() { return D == 64 || D == 128 ? 2 : bwd_group<D>(); }
-template <int D>
-constexpr int dq_waves() { return D == 64 ? 3 : D == 128 ? 2 : bwd_waves<D>(); }
+constexpr int dq_waves() { return D == 64 ? 3 : bwd_waves<D>(); }
+template <int D, int WAVES>
+constexpr int dq_group() { return D == 64 || (D == 128 && WAVES == 2) ? 2 : bwd_group<D>(); }
 
 // The wave index, wave-uniform at D = 64 (so every LDS address derived from it, the direct-to-LDS
 // loads' M0 values among them, is computed in scalar registers instead of VGPRs that the 3-wave dQ
@@ -47,10 +48,10 @@ __device__ __forceinline__ uint16_t* wave_tile(uint16_t (&arr)[2][NG][TE], int w
   return &arr[0][0][0] + wave * TE;
 }
 
-template <int D, class E>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(dq_waves<D>(), 8))) void attn_bwd_dq_kernel(const AttnArgs a) {
+template <int D, class E, int WAVES = dq_waves<D>()>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WAVES, 8))) void attn_bwd_dq_kernel(const AttnArgs a) {
   using G = TileGeom<D>;
-  constexpr int NG = dq_group<D>();
+  constexpr int NG = dq_group<D, WAVES>();
   // Head dims of 64 and more stage K / V blocks by direct global -> LDS loads into dense swizzled
   // tiles (frees the staging VGPRs: -7 % at D = 128, -2 % of the C3 step at D = 64 under the
   // iterative ILP schedule); smaller ones through registers into padded tiles.
@@ -235,7 +236,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(dq_waves<D>
           for (int e = 0; e < 16; ++e) sc[e] = __builtin_fmaf(sc[e], scale2, neg_lse);
           if (!((full2 >> y) & 1))
             mask_partial<EXACT>(sc, lr, ws, t0, g,
-                                [&] { return qs_exact_bits<D == 128 ? 2 : 16>(a, b, lr, plan.stream(i), t0, g, dq_doc); });
+                                [&] { return qs_exact_bits<D == 128 && WAVES == 2 ? 2 : 16>(a, b, lr, plan.stream(i), t0, g, dq_doc); });
           uint32_t dsk[8];
 #pragma unroll
           for (int e = 0; e < 8; ++e) {

@@ -18,7 +18,7 @@
 // (kernel time, MI355X): D = 256, B2 H8 N2048, packed documents, 400-495 -> 109 us; D = 128, B2 H16
 // N4096, 158 -> 138 us; D = 128 f16, B3 H10 N3062, 87 -> 77 us. At D = 64 the one-wave form holds two
 // waves per SIMD by itself and is faster (88 against 96 us at B4 H16 N4096), so it keeps that.
-#include "attn_bwd_dq.hpp"
+#include "attn_tiles.hpp"
 
 namespace sps {
 
@@ -255,15 +255,6 @@ __global__ __launch_bounds__(kSplitThreads) void attn_bwd_dkdv_split_kernel(cons
       for (int ii = 0; ii < 4; ++ii) *reinterpret_cast<u32x2_t*>(orow + 32 * dc + 8 * ii + 4 * g) = piece(dc, ii);
     }
   }
-}
-
-hipError_t launch_attn_bwd_dq_128(const AttnArgs& a, int is_f16, int64_t nblocks, hipStream_t stream) {
-  const dim3 grid((unsigned)nblocks), block(256);
-  if (is_f16)
-    hipLaunchKernelGGL((attn_bwd_dq_kernel<128, ElemF16>), grid, block, 0, stream, a);
-  else
-    hipLaunchKernelGGL((attn_bwd_dq_kernel<128, ElemBF16>), grid, block, 0, stream, a);
-  return hipGetLastError();
 }
 
 hipError_t launch_attn_bwd_dkdv_split(const AttnArgs& a, int D, int is_f16, int64_t nblocks, hipStream_t stream) {

@@ -119,9 +119,7 @@ constexpr int kBwdDkdv = 2;
 hipError_t launch_row_layout(const AttnArgs& a, hipStream_t stream);
 hipError_t launch_attn_fwd(const AttnArgs& a, int D, int is_f16, hipStream_t stream);
 hipError_t launch_attn_bwd(const AttnArgs& a, int D, int is_f16, int passes, hipStream_t stream);
-// The dQ pass at head dim 128, and the dK/dV pass at head dims of 128 and 256 (nblocks workgroups: one
-// per tile, row and head).
-hipError_t launch_attn_bwd_dq_128(const AttnArgs& a, int is_f16, int64_t nblocks, hipStream_t stream);
+// The dK/dV pass at head dims of 128 and 256 (nblocks workgroups: one per tile, row and head).
 hipError_t launch_attn_bwd_dkdv_split(const AttnArgs& a, int D, int is_f16, int64_t nblocks, hipStream_t stream);
 hipError_t launch_mask_dump(const AttnArgs& a, int schedule, hipStream_t stream);
 

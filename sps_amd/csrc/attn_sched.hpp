@@ -231,6 +231,33 @@ __host__ __device__ __forceinline__ int k_tiles(int family, int N, int P) {
   return k_tiles_stream(family, N, STREAM_PERSISTENT, P) + k_tiles_stream(family, N, STREAM_TEMPORARY, P);
 }
 
+// Most 32-key blocks a query tile can need over its streams, whatever the documents: what the windows
+// leave of each stream (a tile spans kTile / 2 tokens), which need not start on a block.
+inline int longest_q_tile(const MaskSpec& m) {
+  if (m.family == FAMILY_FULL) return (m.N + kBlock - 1) / kBlock;
+  auto blocks = [&](int stream, int window) {
+    const int all = (stream_len(m.family, m.N, stream, m.P) + kBlock - 1) / kBlock;
+    return imin(all, (imax(window, 0) + kTile / 2 + kBlock - 1) / kBlock + 1);
+  };
+  return blocks(STREAM_PERSISTENT, m.has_pkw ? m.pkw : m.N) + blocks(STREAM_TEMPORARY, m.window);
+}
+
+// Which form the dQ pass takes at head dim 128, from the sizes the host knows (`tiles`: query tiles over all
+// rows and heads, one workgroup each). Two workgroups on a CU (two waves per SIMD) get through a block
+// ~15 % faster than one, but a workgroup alone on its CU takes up to 9 % longer than in the one-wave form.
+// MI355X, 256 CUs, dQ and in brackets the whole step, two waves against one:
+//  - up to 256 tiles, one on a CU: -1 to +9 % [-1 to +3 %]: one wave.
+//  - past 512 tiles: -22 to +8 % [-9 to +4 %], C4 (1024 tiles) 118.5 -> 107.2 us; of 378 sizes and packed or
+//    dense layouts 7 lose more than 1 % of the step, most of them at 720 tiles of long documents: two waves.
+//  - between, the heaviest tiles of long documents are left alone on their CUs: 512 tiles of 64 blocks at most +3 to
+//    +16 % [-1 to +6 %]. Without documents, or where windows bound the heaviest tile to a twelfth of the
+//    grid's tiles in blocks, the others' work covers it: [-9 to +1 %] (both windows 64 tokens: 288 tiles; 128
+//    and 512: 320; both 512: 512).
+inline bool dq_two_waves(const MaskSpec& m, int64_t tiles) {
+  if (tiles <= 256) return false;
+  return tiles > 512 || !m.has_docs || tiles >= 12 * (int64_t)longest_q_tile(m);
+}
+
 // Stream and first stream index of key tile kt.
 __host__ __device__ __forceinline__ void k_tile_run(const MaskSpec& m, int kt, int& stream, int& first) {
   if (m.family == FAMILY_FULL) {

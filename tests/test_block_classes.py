@@ -65,3 +65,17 @@ def test_fast_division_and_slot_rotation(tmp_path):
     out = subprocess.run([str(exe), "20000"], capture_output=True, text=True, timeout=300)
     assert out.returncode == 0, out.stdout + out.stderr
     assert out.stdout.strip().endswith("bad 0")
+
+
+@pytest.mark.skipif(shutil.which("hipcc") is None and not Path("/opt/rocm/bin/hipcc").exists(),
+                    reason="hipcc not available")
+def test_dq_form_rule(tmp_path):
+    # The dQ pass at head dim 128 picks one wave or two per SIMD from the grid and the longest tile that the
+    # windows allow; the host check compares that bound with the tiles' plans, and the rule with its limits.
+    hipcc = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
+    exe = tmp_path / "dq_form_check"
+    subprocess.run([hipcc, "--offload-arch=gfx950", "-O2", "-std=c++17", "-w",
+                    str(HERE / "native" / "dq_form_check.hip"), "-o", str(exe)], check=True)
+    out = subprocess.run([str(exe), "20000"], capture_output=True, text=True, timeout=300)
+    assert out.returncode == 0, out.stdout + out.stderr
+    assert out.stdout.strip().endswith("bad 0")
