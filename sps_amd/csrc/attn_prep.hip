@@ -144,16 +144,17 @@ __global__ __launch_bounds__(kPrepThreads) void row_layout_kernel(const AttnArgs
   bool flag[kRegIds];
   if (in_regs) {
     // Common case: every id of this thread's chunk (and its predecessor) loaded once, together, in
-    // 16-byte pieces where the row is aligned and the chunk whole, else one by one with positions clamped
-    // into the row (values past the chunk are never used).
+    // 16-byte pieces where the chunk is whole, else one by one with positions clamped into the row (values
+    // past the chunk are never used). The pieces start at an id, wherever it lies: rows of odd lengths are not
+    // 16-byte aligned, and global loads need 4 bytes only.
     int64_t before = 0;
     auto load_all = [&](auto* ids) {
       using T = std::remove_cv_t<std::remove_pointer_t<decltype(ids)>>;
       ids += (int64_t)b * a.docs_sb;
       constexpr int kBytes = kRegIds * (int)sizeof(T), kVec = kBytes < 16 ? kBytes : 16;
-      typedef T vec_t __attribute__((ext_vector_type(kVec / (int)sizeof(T))));
+      typedef T vec_t __attribute__((ext_vector_type(kVec / (int)sizeof(T)), aligned(sizeof(T))));
       const int64_t bv = ids[imax(imin(p0, N) - 1, 0)];
-      if ((reinterpret_cast<uintptr_t>(ids) & (kVec - 1)) == 0 && p0 + kRegIds <= N) {
+      if (p0 + kRegIds <= N) {
         vec_t x[kBytes / kVec];
 #pragma unroll
         for (int v = 0; v < kBytes / kVec; ++v) x[v] = reinterpret_cast<const vec_t*>(ids + p0)[v];
@@ -241,8 +242,10 @@ __global__ __launch_bounds__(kPrepThreads) void row_layout_kernel(const AttnArgs
   if (tid == 0) a.row_mono[b] = mono ? 1 : 0;
   if (in_regs) {
     lds_barrier();  // the plans read only LDS
-    // The global arrays, 4 (2) positions a store where the rows are aligned; the stores drain while the
-    // plans below are computed.
+    // The global arrays; the stores drain while the plans below are computed. Rows the store width divides: the
+    // thread's own positions, 4 (2) a store. Others: consecutive positions of the wave from LDS, since 4-byte stores
+    // of own positions touch a line each (with the ids' loads in pieces, prepass and a one-head forward, B4, N = 7001:
+    // 38.4 -> 31.3 us with int32 ids, 37.0 -> 31.4 with int64).
     constexpr int kStore = kRegIds < 4 ? kRegIds : 4;
     typedef int store_t __attribute__((ext_vector_type(kStore)));
     if ((N & (kStore - 1)) == 0) {
@@ -261,17 +264,15 @@ __global__ __launch_bounds__(kPrepThreads) void row_layout_kernel(const AttnArgs
         }
       }
     } else {
-#pragma unroll
-      for (int j = 0; j < kRegIds; ++j) {
-        if (p0 + j >= N) continue;
-        start[p0 + j] = cs[j];
-        end[p0 + j] = ce[j];
+      for (int p = tid; p < N; p += kPrepThreads) {
+        start[p] = s_start[p];
+        end[p] = s_end[p];
       }
     }
   } else {
     __syncthreads();  // start/end of the whole row are visible to every thread below
   }
-  // Rows that fit read their run bounds from LDS (short: positions < kLdsRow <= 32767).
+  // Rows that fit read their run bounds from LDS (16 bits: positions < kLdsRow <= 8192).
   const bool lds_ok = in_regs;
 
   // Query-tile and key-tile plans, then both sorts. Rows with more than

@@ -29,3 +29,10 @@ def test_runs_and_plans(n, dtype, offset):
         want = torch.from_numpy(np.stack([M.mask_c(family, n, r, window) for r in ids])).cuda()
         for schedule in (0, 1):
             assert torch.equal(SA.attention_mask(family, n, docs, window=window, schedule=schedule), want)
+
+
+@pytest.mark.parametrize("n", [2051, 4097, 4101, 6001, 6002, 8189, 8190, 8191])
+@pytest.mark.parametrize("dtype", [torch.int64, torch.int32])
+def test_rows_no_store_divides(n, dtype):
+    # Run bounds stored from LDS, and ids loaded in pieces from rows that start at any id.
+    test_runs_and_plans(n, dtype, 0)
