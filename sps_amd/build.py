@@ -71,11 +71,16 @@ def _compile(hipcc: str, src: Path, obj: Path) -> None:
 
 
 def _compile_binding(obj: Path) -> None:
-    """The torch binding's object: host code only (g++, torch and HIP headers)."""
+    """The torch binding's object: host code only (g++, torch and HIP headers).
+
+    NDEBUG takes out pybind11's reference-count check, whose counter is thread-local: where a module with
+    thread-local storage is loaded after autograd's threads have started, glibc (2.35) looks every access of theirs
+    to torch's own up on a slow path, which cost each backward of a Python autograd function in the process ~8 us
+    (209 -> 217 us)."""
     from torch.utils import cpp_extension
 
     includes = [*cpp_extension.include_paths(), "/opt/rocm/include", sysconfig.get_paths()["include"]]
-    cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-DUSE_ROCM", "-D__HIP_PLATFORM_AMD__=1",
+    cmd = [os.environ.get("CXX", "g++"), "-O2", "-DNDEBUG", "-std=c++17", "-fPIC", "-DUSE_ROCM", "-D__HIP_PLATFORM_AMD__=1",
            f"-D_GLIBCXX_USE_CXX11_ABI={int(torch.compiled_with_cxx11_abi())}",
            *(f"-isystem{p}" for p in includes), "-c", str(CSRC / "torch_binding.cpp"), "-o", str(obj)]
     proc = subprocess.run(cmd, capture_output=True, text=True)

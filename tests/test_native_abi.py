@@ -4,6 +4,7 @@ GPU is visible: a call whose arguments passed validation could otherwise launch 
 
 import ctypes as C
 import re
+import struct
 from pathlib import Path
 
 import pytest
@@ -17,6 +18,15 @@ def _declared_functions():
     text = HEADER.read_text()
     text = re.sub(r"/\*.*?\*/", "", text, flags=re.S)
     return sorted(set(re.findall(r"\b(sps_[a-z0-9_]+)\s*\(", text)))
+
+
+def test_torch_binding_brings_no_thread_local_storage():
+    # A PT_TLS segment (type 7) in the module slows every access to torch's thread-local state after it is loaded.
+    data = (Path(N.__file__).parent / "_torch_binding.so").read_bytes()
+    assert data[:6] == b"\x7fELF\x02\x01"  # 64 bits, little endian
+    offset, = struct.unpack_from("<Q", data, 32)
+    size, count = struct.unpack_from("<HH", data, 54)
+    assert 7 not in [struct.unpack_from("<I", data, offset + i * size)[0] for i in range(count)]
 
 
 def test_header_declarations_match_binding():
