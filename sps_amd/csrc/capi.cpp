@@ -405,12 +405,7 @@ static int decode_impl(int B, int H, int D, int nq, const void* q, int q_dtype, 
     sg.len_i64 = seg_len_dtype[s] == SPS_DTYPE_I64;
     sg.len_per_head = seg_len_per_head[s] != 0;
   }
-  // Segments with scan 0 own no chunk; give them a valid (never read) length pointer source.
-  for (int s = 0; s < n_seg; ++s) {
-    if (a.seg[s].scan == 0) {
-      a.seg[s].len = nullptr;
-    }
-  }
+  // Segments with scan 0 own no chunk: their pointers stay null, and the merge kernel loads no length of theirs.
   a.n_chunks = chunk;
   a.chunk_keys = ck;
   a.chunk_shift = __builtin_ctz((unsigned)ck);

@@ -11,8 +11,9 @@
 //
 // Every function here takes only the calls whose handling needs nothing but the kernels: exact
 // torch.Tensor / Parameter arguments on one GPU, in the types, layouts and shapes the kernels read in
-// place, with no dispatch or function mode, functorch transform, tracer or forward-mode dual number
-// about. For any other call it returns None before doing anything, and the Python caller takes its
+// place, with no dispatch or function mode (torch.set_default_device is one), functorch transform, tracer or
+// forward-mode dual number about; with gradients, q, k and v (and RoPE's frequencies) also have to be dense, so
+// slices of one projection go the general way there. For any other call it returns None before doing anything, and the Python caller takes its
 // general path (the torch.library ops, conversions, error messages), so nothing here raises for a
 // malformed argument. The autograd functions save tensors through the ordinary hooks and, where their
 // backward meets such a case (create_graph, batched gradients), call the same torch.library ops.
