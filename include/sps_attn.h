@@ -330,7 +330,8 @@ int sps_prefill_to_decode(int B, int T, int H, int D, int in_dtype, const void* 
  * 2) times: out[b, t * repeat + r], int32/int64 with row stride out_stride_b (repeat = 2 gives the
  * [B, 2T] ids of the interleaved input/<predict> sequence). Rows must be left padded: bad_rows
  * (int32 [B], may be null) receives 1 for a row with a pad token after a real token (its ids follow
- * the same formula; the reference raises ValueError for such input) and 0 otherwise.
+ * the same formula; the reference raises ValueError for such input) and 0 otherwise. With T == 0
+ * nothing is launched or written, bad_rows included.
  */
 int sps_document_ids(int B, int T, const void* tokens, int tokens_dtype, int64_t tokens_stride_b,
                      int64_t eos_token_id, int64_t pad_token_id, int repeat, void* out, int out_dtype,
